@@ -2,13 +2,15 @@
 // gfx950 matrix cores (see mlp.hpp for the network and operand layouts).
 //
 // Training step on a minibatch of B rows (all kernels hand-written):
-//   forward   Z_l = A_{l-1} W_l + b_l, A_l = bf16(silu(Z_l))   (k_gemm FWD)
-//   loss      dY = bf16(2 (Y - T) / (8 B)), per-row squared error (k_loss)
-//   backward  dZ_{l-1} = bf16((dZ_l W_l^T) * silu'(Z_{l-1}))     (k_gemm BWD)
-//             partial dW_l = A_{l-1}^T dZ_l over row chunks        (k_gemm WGRAD)
-//             partial db_l = column sums of dZ_l over row chunks   (k_colsum)
-//   update    sum the chunk partials in a fixed order, Adam on the FP32
-//             master weights, refresh the BF16 copies           (k_adam)
+//   k_train_rows   a wave takes 16 rows forward and back in registers: each
+//                  layer's accumulators, through SiLU and BF16, are the next
+//                  layer's MFMA operand in both directions.  It leaves every
+//                  layer's activations and dZ as the operands of the weight
+//                  gradient, and the per-row squared errors.
+//   k_train_wgrad  dW_l = A_{l-1}^T dZ_l and db_l of a chunk of rows, all
+//                  layers, straight from those operands
+//   k_train_update sum the chunks in a fixed order, Adam on the FP32 master
+//                  weights, refresh the BF16 operand copies
 // Every reduction has a fixed order, so a training run is deterministic.
 // Inference (k_infer) keeps all 58 KiB of fragment-ordered BF16 weights in
 // LDS and pushes 16-row tiles through the four layers per wavefront.
@@ -28,137 +30,347 @@ using namespace bats::mlp;
 
 namespace {
 
-enum { EPI_FWD = 0, EPI_OUT = 1, EPI_BWD = 2, EPI_WGRAD = 3 };
+// ---- training step ------------------------------------------------------
+// Operands of the weight gradient.  Its MFMAs sum over rows, so a lane needs
+// one feature at several rows, while a row's own chain holds one row at
+// several features.  The matrix cores turn the one into the other: an
+// activation fragment as the A operand times a unit matrix gives its 16 x 16
+// blocks with a lane holding feature l%16 at rows 4 (l/16) .. +3, exactly
+// (each sum has one term).  A 16-row tile leaves NTB blocks of 64 lanes x 4
+// values; two consecutive tiles make a 32-row operand.
+constexpr int TB_A0 = 0, TB_A1 = 1, TB_A2 = 9, TB_A3 = 17;   // X, A1, A2, A3
+constexpr int TB_Z1 = 21, TB_Z2 = 29, TB_Z3 = 37, TB_Z4 = 41; // dZ1..dZ3, dY
+constexpr int NTB = 42;
+constexpr int kTrainThreads = 512, kTrainWaves = kTrainThreads / 64;
 
-struct GemmArgs {
-  int M, N, K;
-  const __bf16 *A;  // A(m,k) = A[m*sAm + k*sAk]
-  long sAm, sAk;
-  const __bf16 *B;  // B(k,n) = B[k*sBk + n*sBn]
-  long sBk, sBn;
-  const float *bias;     // FWD/OUT: [N]
-  float *Cf;             // FWD: Z, OUT: Y, WGRAD: partial (ld = ldc)
-  long ldc;
-  __bf16 *Cb;            // FWD: A = silu(Z), BWD: dZ (ld = ldc)
-  const float *Zprev;    // BWD: pre-activation of the layer below (ld = ldc)
-  int kChunk;            // WGRAD: rows per split (blockIdx.y)
-  long partialStride;    // WGRAD: floats between splits
+struct TrainArgs {
+  const __bf16 *frag, *bfrag;  // weights, fragment order
+  const float *w;              // flat FP32 parameters (biases)
+  const float *X, *T;          // samples: inputs and targets
+  const float *J;              // target weights or null
+  float invMeanJ;
+  const float *scale;          // targets are divided by scale[j] (or null)
+  const int *idx;              // rows of the minibatch (null: 0 .. B-1);
+  long perEpoch;               // step q takes idx[(q % perEpoch) * B ...]
+  long *step;                  // [0] this step's number, copied to [1]
+  int B;
+  bf16x4 *ops;                 // [tile][NTB][64]
+  float *rowErr;
 };
 
-// one 16x16 output tile per wavefront, K in steps of 32
-template <int EPI>
-__global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
-  const int lane = threadIdx.x & 63;
-  const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int nTn = (g.N + 15) / 16;
-  const int m0 = (tile / nTn) * 16, n0 = (tile % nTn) * 16;
-  if (m0 >= g.M) return;  // wave-uniform
-  int kBeg = 0, kEnd = g.K;
-  if (EPI == EPI_WGRAD) {
-    kBeg = blockIdx.y * g.kChunk;
-    kEnd = min(g.K, kBeg + g.kChunk);
-  }
-  const int r = lane & 15, kq = 8 * (lane >> 4);
-  const int am = m0 + r, bn = n0 + r;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = kBeg; k0 < kEnd; k0 += 32) {
-    bf16x8 a, b;
+// One pass instead of a matrix product per layer and direction: at 65,536
+// rows a training step (this, k_train_wgrad, k_train_update) takes 34 + 26 +
+// 8 us where 17 kernels with the activations in memory between them took
+// 560 us.  Bound by the vector unit (two transcendentals and about 20
+// instructions per activation for SiLU, its derivative and the roundings)
+// and by the 21.5 KB per tile it stores (88 MB, 18 us at the card's copy
+// rate); the weights of both directions stay in LDS (110 KiB, one workgroup
+// per CU, two waves per SIMD).
+__global__ void __launch_bounds__(kTrainThreads)
+k_train_rows(TrainArgs a) {
+  __shared__ __attribute__((aligned(16))) __bf16 sW[NFRAG];
+  __shared__ __attribute__((aligned(16))) __bf16 sB[NBFRAG];
+  __shared__ float sBias[NBIAS];
+  for (int t = threadIdx.x; t < NFRAG / 8; t += kTrainThreads)
+    reinterpret_cast<bf16x8 *>(sW)[t] =
+        reinterpret_cast<const bf16x8 *>(a.frag)[t];
+  for (int t = threadIdx.x; t < NBFRAG / 8; t += kTrainThreads)
+    reinterpret_cast<bf16x8 *>(sB)[t] =
+        reinterpret_cast<const bf16x8 *>(a.bfrag)[t];
+  load_biases(a.w, sBias);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const bf16x8 *W = reinterpret_cast<const bf16x8 *>(sW) + lane;
+  const bf16x8 *V = reinterpret_cast<const bf16x8 *>(sB) + lane;
+  const long q = a.step ? a.step[0] : 0;
+  if (a.step && blockIdx.x == 0 && threadIdx.x == 0) a.step[1] = q;
+  const int *idx = a.idx ? a.idx + (q % a.perEpoch) * a.B : nullptr;
+  // unit blocks in the slot orders of frag_k: natural (the inputs), and the
+  // two 16-feature halves of an accumulator fragment
+  bf16x8 unitX, unit[2];
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
-      const int k = k0 + kq + t;
-      const bool ok = k < kEnd;
-      a[t] = (ok && am < g.M) ? g.A[am * g.sAm + k * g.sAk] : (__bf16)0.0f;
-      b[t] = (ok && bn < g.N) ? g.B[k * g.sBk + bn * g.sBn] : (__bf16)0.0f;
-    }
-    acc = mfma(a, b, acc);
+  for (int t = 0; t < 8; t++) {
+    unitX[t] = (__bf16)(8 * g + t == r ? 1.f : 0.f);
+    unit[0][t] = (__bf16)(t < 4 && 4 * g + t == r ? 1.f : 0.f);
+    unit[1][t] = (__bf16)(t >= 4 && 4 * g + t - 4 == r ? 1.f : 0.f);
   }
-  const int n = n0 + r;
-  if (n >= g.N) return;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  // an even number of tiles: two make an operand of k_train_wgrad
+  const int nTile = (a.B + 31) / 32 * 2;
+  for (int tile = blockIdx.x * kTrainWaves + (threadIdx.x >> 6); tile < nTile;
+       tile += gridDim.x * kTrainWaves) {
+    const int row = tile * 16 + r;
+    const bool ok = row < a.B;
+    const long s = ok ? (idx ? idx[row] : row) : 0;
+    bf16x4 *ops = a.ops + (long)tile * NTB * 64 + lane;
+    auto turn = [&](bf16x8 x, bf16x8 u, int block) {
+      const f32x4 d = mfma(x, u, zero);
+      bf16x4 o;
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int m = m0 + 4 * (lane >> 4) + i;
-    if (m >= g.M) continue;
-    const float v = acc[i];
-    if (EPI == EPI_FWD) {
-      const float z = v + g.bias[n];
-      g.Cf[m * g.ldc + n] = z;
-      g.Cb[m * g.ldc + n] = (__bf16)silu(z);
-    } else if (EPI == EPI_OUT) {
-      g.Cf[m * g.ldc + n] = v + g.bias[n];
-    } else if (EPI == EPI_BWD) {
-      g.Cb[m * g.ldc + n] = (__bf16)(v * dsilu(g.Zprev[m * g.ldc + n]));
-    } else {
-      g.Cf[blockIdx.y * g.partialStride + m * g.ldc + n] = v;
+      for (int i = 0; i < 4; i++) o[i] = (__bf16)d[i];
+      ops[block * 64] = o;
+    };
+    auto turn2 = [&](bf16x8 x, int block) {
+      turn(x, unit[0], block);
+      turn(x, unit[1], block + 1);
+    };
+    bf16x8 x;
+#pragma unroll
+    for (int t = 0; t < 8; t++)
+      x[t] = (ok && g < 2) ? (__bf16)a.X[s * 16 + 8 * g + t] : (__bf16)0.f;
+    turn(x, unitX, TB_A0);
+    // forward: z = W^T a + b, a' = bf16(silu(z)); the derivative silu'(z)
+    // of every unit stays in registers for the way back
+    f32x4 acc[8], d1[8], d2[8], d3[4];
+    bf16x8 f[4];
+    auto act = [&](f32x4 *d, const float *b, int nb2, bf16x8 *o, int block) {
+#pragma unroll
+      for (int kb = 0; kb < nb2; kb++) {
+        bf16x8 v;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          const int nb = 2 * kb + h;
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const float z = acc[nb][i] + b[nb * 16 + 4 * g + i];
+            const float sg = sigmoid(z);
+            v[4 * h + i] = (__bf16)(z * sg);
+            d[nb][i] = sg * (1.0f + z * (1.0f - sg));
+          }
+        }
+        o[kb] = v;
+        turn2(v, block + 2 * kb);
+      }
+    };
+#pragma unroll
+    for (int nb = 0; nb < 8; nb++) acc[nb] = mfma(W[(FT0 + nb) * 64], x, zero);
+    act(d1, sBias + CB1, 4, f, TB_A1);
+#pragma unroll
+    for (int nb = 0; nb < 8; nb++) {
+      acc[nb] = zero;
+#pragma unroll
+      for (int kb = 0; kb < 4; kb++)
+        acc[nb] = mfma(W[(FT1 + nb * 4 + kb) * 64], f[kb], acc[nb]);
+      __builtin_amdgcn_sched_barrier(0);
     }
+    act(d2, sBias + CB2, 4, f, TB_A2);
+#pragma unroll
+    for (int nb = 0; nb < 4; nb++) {
+      acc[nb] = zero;
+#pragma unroll
+      for (int kb = 0; kb < 4; kb++)
+        acc[nb] = mfma(W[(FT2 + nb * 4 + kb) * 64], f[kb], acc[nb]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    act(d3, sBias + CB3, 2, f, TB_A3);
+    f32x4 y = mfma(W[(FT3 + 0) * 64], f[0], zero);
+    y = mfma(W[(FT3 + 1) * 64], f[1], y);
+    // loss (1/(8B)) sum_r W_r |Y_r - T_r|^2: the error of a row summed over
+    // its outputs in order (lanes g = 0, then g = 1), and dY
+    bf16x8 z4 = {};
+    float dj[4], sq = 0.f;
+    const float wr = (a.J && ok) ? a.J[s] * a.invMeanJ : 1.0f;
+    const float sc = 2.0f * wr / (8.0f * (float)a.B);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int n = 4 * g + i;
+      float t = (ok && g < 2) ? a.T[s * 8 + n] : 0.f;
+      if (a.scale && g < 2) t = t / a.scale[n];
+      dj[i] = (ok && g < 2) ? y[i] + sBias[CB4 + (g < 2 ? n : 0)] - t : 0.f;
+      z4[i] = (__bf16)(sc * dj[i]);
+    }
+    if (g == 0)
+#pragma unroll
+      for (int i = 0; i < 4; i++) sq += dj[i] * dj[i];
+    const float first = __shfl(sq, r, 64);
+    if (g == 1 && ok) {
+      sq = first;
+#pragma unroll
+      for (int i = 0; i < 4; i++) sq += dj[i] * dj[i];
+      a.rowErr[row] = wr * sq;
+    }
+    turn(z4, unit[0], TB_Z4);
+    // back: dZ = bf16((W dZ') silu'(z))
+    auto back = [&](const f32x4 *d, int nb2, bf16x8 *o, int block) {
+#pragma unroll
+      for (int kb = 0; kb < nb2; kb++) {
+        bf16x8 v;
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            v[4 * h + i] = (__bf16)(acc[2 * kb + h][i] * d[2 * kb + h][i]);
+        o[kb] = v;
+        turn2(v, block + 2 * kb);
+      }
+    };
+#pragma unroll
+    for (int mb = 0; mb < 4; mb++) acc[mb] = mfma(V[(BT3 + mb) * 64], z4, zero);
+    back(d3, 2, f, TB_Z3);
+#pragma unroll
+    for (int mb = 0; mb < 8; mb++) {
+      acc[mb] = zero;
+#pragma unroll
+      for (int kb = 0; kb < 2; kb++)
+        acc[mb] = mfma(V[(BT2 + mb * 2 + kb) * 64], f[kb], acc[mb]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    back(d2, 4, f, TB_Z2);
+#pragma unroll
+    for (int mb = 0; mb < 8; mb++) {
+      acc[mb] = zero;
+#pragma unroll
+      for (int kb = 0; kb < 4; kb++)
+        acc[mb] = mfma(V[(BT1 + mb * 4 + kb) * 64], f[kb], acc[mb]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    back(d1, 4, f, TB_Z1);
   }
 }
 
-// dY = bf16(2 (Y - T) / (8 B)); per-row squared error sums
-// loss (1/(8B)) sum_r W_r |Y_r - T_r|^2 (W null: all one), its gradient
-// dY and the per-row squared errors W_r |Y_r - T_r|^2
-__global__ void k_loss(const float *Y, const float *T, const float *W, int B,
-                       __bf16 *dY, float *rowErr) {
-  const int row = blockIdx.x * blockDim.x + threadIdx.x;
-  if (row >= B) return;
-  float s = 0.f;
-  const float wr = W ? W[row] : 1.0f;
-  const float sc = 2.0f * wr / (8.0f * (float)B);
-  for (int j = 0; j < 8; j++) {
-    const float d = Y[row * 8 + j] - T[row * 8 + j];
-    s += d * d;
-    dY[row * 8 + j] = (__bf16)(sc * d);
+// Weight and bias gradients of a chunk of rows (blockIdx.x): the four waves
+// share the 108 weight tiles and the 21 bias tiles (a unit row of ones times
+// dZ); every operand is 512 contiguous bytes per 16 rows, read once per wave
+// that needs it (84 KB per 32 rows and workgroup, 42 KB of it distinct).
+// Bound by reading them: 26 us for 88 MB at 65,536 rows.
+__global__ void __launch_bounds__(256)
+k_train_wgrad(const bf16x4 *ops, int nPair, int perChunk, float *partial,
+              long *step) {
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int wv = threadIdx.x >> 6;
+  if (step && blockIdx.x == 0 && threadIdx.x == 0) step[0] = step[1] + 1;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 w1[2], w2[2][8], w3[2][4], w4 = zero, b1[2], b2[2], b3 = zero, b4 = zero;
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    w1[i] = b1[i] = b2[i] = zero;
+    for (int n = 0; n < 8; n++) w2[i][n] = zero;
+    for (int n = 0; n < 4; n++) w3[i][n] = zero;
   }
-  rowErr[row] = wr * s;
+  bf16x8 ones;
+#pragma unroll
+  for (int t = 0; t < 8; t++) ones[t] = (__bf16)1.0f;
+  const int p0 = blockIdx.x * perChunk;
+  const int p1 = p0 + perChunk < nPair ? p0 + perChunk : nPair;
+  for (int p = p0; p < p1; p++) {
+    const bf16x4 *o = ops + (long)p * 2 * NTB * 64 + lane;
+    auto op = [&](int block) {
+      const bf16x4 lo = o[block * 64], hi = o[(NTB + block) * 64];
+      return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    const bf16x8 x = op(TB_A0);
+    bf16x8 z[8], c[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      c[i] = op(TB_Z1 + 2 * wv + i);
+      w1[i] = mfma(x, c[i], w1[i]);
+      b1[i] = mfma(ones, c[i], b1[i]);
+    }
+#pragma unroll
+    for (int n = 0; n < 8; n++) z[n] = op(TB_Z2 + n);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      c[i] = op(TB_A1 + 2 * wv + i);
+#pragma unroll
+      for (int n = 0; n < 8; n++) w2[i][n] = mfma(c[i], z[n], w2[i][n]);
+    }
+    // (a register array indexed by the wave would go to memory)
+    b2[0] = mfma(ones, op(TB_Z2 + 2 * wv), b2[0]);
+    b2[1] = mfma(ones, op(TB_Z2 + 2 * wv + 1), b2[1]);
+#pragma unroll
+    for (int n = 0; n < 4; n++) z[n] = op(TB_Z3 + n);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      c[i] = op(TB_A2 + 2 * wv + i);
+#pragma unroll
+      for (int n = 0; n < 4; n++) w3[i][n] = mfma(c[i], z[n], w3[i][n]);
+    }
+    b3 = mfma(ones, op(TB_Z3 + wv), b3);
+    const bf16x8 y = op(TB_Z4);
+    w4 = mfma(op(TB_A3 + wv), y, w4);
+    b4 = mfma(ones, y, b4);
+  }
+  // tile (m, n): lane holds column n = l%16, rows m = 4 (l/16) + i
+  float *P = partial + (long)blockIdx.x * NPARAM;
+  auto put = [&](int l, int mb, int nb, f32x4 v) {
+    const int n = nb * 16 + r;
+    if (n < DIM[l + 1])
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        P[OW[l] + (mb * 16 + 4 * g + i) * DIM[l + 1] + n] = v[i];
+  };
+  auto putb = [&](int l, int nb, f32x4 v) {
+    const int n = nb * 16 + r;
+    if (g == 0 && n < DIM[l + 1]) P[OB[l] + n] = v[0];
+  };
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    put(0, 0, 2 * wv + i, w1[i]);
+    putb(0, 2 * wv + i, b1[i]);
+#pragma unroll
+    for (int n = 0; n < 8; n++) put(1, 2 * wv + i, n, w2[i][n]);
+    putb(1, 2 * wv + i, b2[i]);
+#pragma unroll
+    for (int n = 0; n < 4; n++) put(2, 2 * wv + i, n, w3[i][n]);
+  }
+  putb(2, wv, b3);
+  put(3, wv, 0, w4);
+  if (wv == 0) putb(3, 0, b4);
 }
 
-// partial column sums of a BF16 [rows x N] matrix over row chunks
-__global__ void k_colsum(const __bf16 *X, int rows, int N, int chunk,
-                         float *partial, long partialStride, int off) {
-  const int n = threadIdx.x;  // N <= 256
-  if (n >= N) return;
-  const int r0 = blockIdx.x * chunk, r1 = min(rows, r0 + chunk);
-  float s = 0.f;
-  for (int r = r0; r < r1; r++) s += (float)X[(long)r * N + n];
-  partial[blockIdx.x * partialStride + off + n] = s;
-}
-
-// gradient = sum of the row-chunk partials, in chunk order
-__global__ void k_sum_partials(const float *partial, int nSplit, float *grad) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= NPARAM) return;
-  float g = 0.f;
-  for (int s = 0; s < nSplit; s++) g += partial[(long)s * NPARAM + p];
-  grad[p] = g;
-}
-
-struct AdamArgs {
-  const float *grad;
+struct UpdateArgs {
+  const float *partial;  // [chunk][NPARAM]
+  int nChunk;
+  float *grad;
+  int adam;              // 0: the gradient only
   float *w, *m, *v;
-  __bf16 *wb;            // BF16 copy, flat layout
-  float lr, b1, b2, eps, bc1, bc2;  // bc = 1 - beta^t
-  // with a schedule (graph-captured training): lr, bc1, bc2 of step
-  // *step are sched[3 * *step + 0..2]
+  __bf16 *frag, *bfrag;  // BF16 operand copies of the weights
+  float b1, b2, eps;
+  // lr, 1 - b1^t, 1 - b2^t of step step[1] are sched[3 * step[1] + 0..2]
   const float *sched;
   const long *step;
 };
 
-// Adam (Kingma & Ba 2015) on the FP32 master weights
-__global__ void k_adam(AdamArgs a) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= NPARAM) return;
-  float lr = a.lr, bc1 = a.bc1, bc2 = a.bc2;
-  if (a.sched) {
-    const float *q = a.sched + 3 * *a.step;
-    lr = q[0]; bc1 = q[1]; bc2 = q[2];
+// gradient = sum of the chunks' partials (eight runs of chunks, each in
+// order, then their sums in order), and Adam (Kingma & Ba 2015) on the FP32
+// master weights.  Bound by reading the partials (28 MB at 256 chunks): 128
+// parameters per workgroup, 16-byte loads, eight of them in flight.
+constexpr int kUpdateParams = 128;
+static_assert(NPARAM % 4 == 0, "partials are read four at a time");
+__global__ void __launch_bounds__(256) k_train_update(UpdateArgs a) {
+  __shared__ float sSum[8][kUpdateParams];
+  const int c = 4 * (threadIdx.x & 31), run = threadIdx.x >> 5;
+  const int p4 = blockIdx.x * kUpdateParams + c;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  const int n0 = a.nChunk * run / 8, n1 = a.nChunk * (run + 1) / 8;
+  if (p4 < NPARAM) {
+#pragma unroll 8
+    for (int n = n0; n < n1; n++)
+      s += *reinterpret_cast<const f32x4 *>(a.partial + (long)n * NPARAM + p4);
   }
-  const float g = a.grad[p];
+  *reinterpret_cast<f32x4 *>(&sSum[run][c]) = s;
+  __syncthreads();
+  const int p = blockIdx.x * kUpdateParams + threadIdx.x;
+  if (threadIdx.x >= kUpdateParams || p >= NPARAM) return;
+  float g = 0.f;
+#pragma unroll
+  for (int q = 0; q < 8; q++) g += sSum[q][threadIdx.x];
+  a.grad[p] = g;
+  if (!a.adam) return;
+  const float *q = a.sched + 3 * a.step[1];
+  const float lr = q[0], bc1 = q[1], bc2 = q[2];
   const float m = a.b1 * a.m[p] + (1.f - a.b1) * g;
   const float v = a.b2 * a.v[p] + (1.f - a.b2) * g * g;
   a.m[p] = m;
   a.v[p] = v;
   const float w = a.w[p] - lr * (m / bc1) / (sqrtf(v / bc2) + a.eps);
   a.w[p] = w;
-  a.wb[p] = (__bf16)w;
+  int l = 0;
+  while (l + 1 < NL && p >= OW[l + 1]) l++;
+  if (p >= OB[l]) return;  // a bias
+  const int k = (p - OW[l]) / DIM[l + 1], n = (p - OW[l]) % DIM[l + 1];
+  a.frag[frag_pos(l, k, n)] = (__bf16)w;
+  if (l > 0) a.bfrag[bfrag_pos(l, k, n)] = (__bf16)w;
 }
 
 // per-block partial sums of squares of the 8 target columns (fixed order)
@@ -188,24 +400,31 @@ __global__ void k_scale_last(float *w, const float *scale, int div) {
   }
 }
 
-__global__ void k_to_bf16(const float *x, __bf16 *y, long n) {
-  const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (t < n) y[t] = (__bf16)x[t];
-}
-
-// fragment-ordered, zero-padded BF16 weights for k_infer
-__global__ void k_pack_frag(const float *w, __bf16 *frag) {
+// fragment-ordered, zero-padded BF16 weights of both directions
+__global__ void k_pack_frag(const float *w, __bf16 *frag, __bf16 *bfrag) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= NFRAG) return;
-  const int tile = t / TILE, lane = (t % TILE) / 8, e = t % 8;
-  int l = 0;
-  while (l + 1 < NL && tile >= FT[l + 1]) l++;
-  const int lt = tile - FT[l], nKb = KP[l] / 32;
-  const int nb = lt / nKb, kb = lt % nKb;
-  const int k = frag_k(l, kb, lane >> 4, e), n = nb * 16 + (lane & 15);
-  const float v = (k < DIM[l] && n < DIM[l + 1])
-                      ? w[OW[l] + k * DIM[l + 1] + n] : 0.0f;
-  frag[t] = (__bf16)v;
+  const int lane = (t % TILE) / 8, e = t % 8;
+  if (t < NFRAG) {
+    const int tile = t / TILE;
+    int l = 0;
+    while (l + 1 < NL && tile >= FT[l + 1]) l++;
+    const int lt = tile - FT[l], nKb = KP[l] / 32;
+    const int nb = lt / nKb, kb = lt % nKb;
+    const int k = frag_k(l, kb, lane >> 4, e), n = nb * 16 + (lane & 15);
+    const float v = (k < DIM[l] && n < DIM[l + 1])
+                        ? w[OW[l] + k * DIM[l + 1] + n] : 0.0f;
+    frag[t] = (__bf16)v;
+  }
+  if (t < NBFRAG) {
+    const int tile = t / TILE;
+    int l = 1;
+    while (l + 1 < NL && tile >= BT[l + 1]) l++;
+    const int lt = tile - BT[l], nKb = l == 3 ? 1 : DIM[l + 1] / 32;
+    const int k = (lt / nKb) * 16 + (lane & 15);
+    const int n = frag_k(1, lt % nKb, lane >> 4, e);
+    const float v = n < DIM[l + 1] ? w[OW[l] + k * DIM[l + 1] + n] : 0.0f;
+    bfrag[t] = (__bf16)v;
+  }
 }
 
 }  // namespace
@@ -229,23 +448,6 @@ k_infer(const __bf16 *frag, const float *w, const float *X, float *Y,
     infer_tile(sW, sBias, X, rows, tile * 16, out);
 }
 
-// minibatch gather: rows idx[0..B) of the dataset into X (BF16) and the
-// standardized targets T / scale
-// a minibatch: inputs (BF16), targets divided by scale, and (W non-null)
-// the loss weights dataJ / meanJ.  With step non-null the rows are
-// idx[(*step % perEpoch) * B + t] (graph-captured training).
-__global__ void k_gather_rows(const float *dataX, const float *dataT,
-                              const int *idx, int B, __bf16 *X, float *T,
-                              const float *scale, const float *dataJ,
-                              float invMeanJ, float *W, const long *step,
-                              long perEpoch) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= B) return;
-  const long s = step ? idx[(*step % perEpoch) * B + t] : idx[t];
-  for (int j = 0; j < 16; j++) X[t * 16 + j] = (__bf16)dataX[s * 16 + j];
-  for (int j = 0; j < 8; j++) T[t * 8 + j] = dataT[s * 8 + j] / scale[j];
-  if (W) W[t] = dataJ[s] * invMeanJ;
-}
 __global__ void k_gather_rows_f32(const float *dataX, const float *dataT,
                                   const float *dataB, const float *dataJ,
                                   const int *idx, int B, float *X, float *T,
@@ -268,16 +470,13 @@ struct bats_mlp {
   hipStream_t stream;
   int dev;                   // device the model (and its stream) lives on
   float *w, *m, *v, *grad;   // FP32 master weights, Adam moments, gradient
-  __bf16 *wb;                // BF16 copy of w (flat layout)
-  __bf16 *frag;              // fragment-ordered BF16 weights for inference
+  __bf16 *frag, *bfrag;      // fragment-ordered BF16 weights, both directions
   int step;                  // Adam steps taken
-  int fragStale;             // frag lags w (repacked before inference)
+  int fragStale;             // frag, bfrag lag w (repacked before use)
   // training buffers for a minibatch of cap rows
   int cap;
-  __bf16 *X, *A1, *A2, *A3, *dZ1, *dZ2, *dZ3, *dY;
-  float *Z1, *Z2, *Z3, *Y, *T, *rowErr, *partial;
-  float *rowW;               // loss weights of the minibatch rows or null
-  int nSplit;
+  bf16x4 *ops;               // weight-gradient operands
+  float *X, *T, *rowErr, *partial;
   // dataset (device): inputs (n x 16), targets (n x 8) and the baseline
   // flux the target corrects (n x 8, zero unless harvested), FP32
   float *dataX, *dataT, *dataB, *dataJ;  // + weight of each sample's target
@@ -294,7 +493,12 @@ struct bats_mlp {
     }                                                                    \
   } while (0)
 
-static const int kChunkRows = 256;  // rows per weight-gradient split
+// row pairs of tiles (32 rows) per weight-gradient chunk: 256 chunks, one
+// per CU, up to 256 rows each
+static int chunk_pairs(int nPair) {
+  const int n = (nPair + 255) / 256;
+  return n < 8 ? n : 8;
+}
 
 // ---- staging memory of bats_mlp_forward_noalloc -----------------------
 // bats_mlp_forward allocates device buffers for the rows it stages in and
@@ -338,18 +542,9 @@ static float *noalloc_scratch(int dev) {
 static int repack(bats_mlp *m) {
   if (!m->fragStale) return BATS_OK;
   hipLaunchKernelGGL(k_pack_frag, dim3((NFRAG + 255) / 256), dim3(256), 0,
-                     m->stream, m->w, m->frag);
+                     m->stream, m->w, m->frag, m->bfrag);
   MCHK(hipGetLastError());
   m->fragStale = 0;
-  return BATS_OK;
-}
-
-static int refresh_copies(bats_mlp *m) {
-  hipLaunchKernelGGL(k_to_bf16, dim3((NPARAM + 255) / 256), dim3(256), 0,
-                     m->stream, m->w, m->wb, (long)NPARAM);
-  hipLaunchKernelGGL(k_pack_frag, dim3((NFRAG + 255) / 256), dim3(256), 0,
-                     m->stream, m->w, m->frag);
-  MCHK(hipGetLastError());
   return BATS_OK;
 }
 
@@ -371,25 +566,23 @@ extern "C" int bats_mlp_create(bats_mlp **out) {
   MCHK(hipMalloc(&m->m, sizeof(float) * NPARAM));
   MCHK(hipMalloc(&m->v, sizeof(float) * NPARAM));
   MCHK(hipMalloc(&m->grad, sizeof(float) * NPARAM));
-  MCHK(hipMalloc(&m->wb, sizeof(__bf16) * NPARAM));
   MCHK(hipMalloc(&m->frag, sizeof(__bf16) * NFRAG));
+  MCHK(hipMalloc(&m->bfrag, sizeof(__bf16) * NBFRAG));
   MCHK(hipMemset(m->w, 0, sizeof(float) * NPARAM));
   MCHK(hipMemset(m->m, 0, sizeof(float) * NPARAM));
   MCHK(hipMemset(m->v, 0, sizeof(float) * NPARAM));
   MCHK(hipMemset(m->grad, 0, sizeof(float) * NPARAM));
   *out = m;
-  return refresh_copies(m);
+  m->fragStale = 1;
+  return repack(m);
 }
 
 static void free_batch(bats_mlp *m) {
-  void *p[] = {m->X, m->A1, m->A2, m->A3, m->dZ1, m->dZ2, m->dZ3, m->dY,
-               m->Z1, m->Z2, m->Z3, m->Y, m->T, m->rowErr, m->partial,
-               m->rowW};
+  void *p[] = {m->ops, m->X, m->T, m->rowErr, m->partial};
   for (void *q : p)
     if (q) (void)hipFree(q);
-  m->X = m->A1 = m->A2 = m->A3 = m->dZ1 = m->dZ2 = m->dZ3 = m->dY = nullptr;
-  m->Z1 = m->Z2 = m->Z3 = m->Y = m->T = m->rowErr = m->partial = nullptr;
-  m->rowW = nullptr;
+  m->ops = nullptr;
+  m->X = m->T = m->rowErr = m->partial = nullptr;
   m->cap = 0;
 }
 
@@ -397,7 +590,7 @@ extern "C" int bats_mlp_free(bats_mlp *m) {
   if (!m) return BATS_EINVAL;
   (void)hipStreamSynchronize(m->stream);
   free_batch(m);
-  void *p[] = {m->w, m->m, m->v, m->grad, m->wb, m->frag, m->dataX, m->dataT,
+  void *p[] = {m->w, m->m, m->v, m->grad, m->frag, m->bfrag, m->dataX, m->dataT,
                m->dataB, m->dataJ};
   for (void *q : p)
     if (q) (void)hipFree(q);
@@ -413,7 +606,8 @@ extern "C" int bats_mlp_set_params(bats_mlp *m, const float *w) {
   MCHK(hipMemsetAsync(m->m, 0, sizeof(float) * NPARAM, m->stream));
   MCHK(hipMemsetAsync(m->v, 0, sizeof(float) * NPARAM, m->stream));
   m->step = 0;
-  int st = refresh_copies(m);
+  m->fragStale = 1;
+  int st = repack(m);
   if (st) return st;
   MCHK(hipStreamSynchronize(m->stream));
   return BATS_OK;
@@ -428,145 +622,73 @@ extern "C" int bats_mlp_get_params(bats_mlp *m, float *w, float *grad) {
   return BATS_OK;
 }
 
+// training buffers for a minibatch of B rows (X and T: the rows that
+// bats_mlp_loss_grad takes from the host)
 static int ensure_batch(bats_mlp *m, int B) {
   if (B <= m->cap) return BATS_OK;
   free_batch(m);
   const size_t b = (size_t)B;
-  MCHK(hipMalloc(&m->X, sizeof(__bf16) * b * 16));
-  MCHK(hipMalloc(&m->A1, sizeof(__bf16) * b * 128));
-  MCHK(hipMalloc(&m->A2, sizeof(__bf16) * b * 128));
-  MCHK(hipMalloc(&m->A3, sizeof(__bf16) * b * 64));
-  MCHK(hipMalloc(&m->dZ1, sizeof(__bf16) * b * 128));
-  MCHK(hipMalloc(&m->dZ2, sizeof(__bf16) * b * 128));
-  MCHK(hipMalloc(&m->dZ3, sizeof(__bf16) * b * 64));
-  MCHK(hipMalloc(&m->dY, sizeof(__bf16) * b * 8));
-  MCHK(hipMalloc(&m->Z1, sizeof(float) * b * 128));
-  MCHK(hipMalloc(&m->Z2, sizeof(float) * b * 128));
-  MCHK(hipMalloc(&m->Z3, sizeof(float) * b * 64));
-  MCHK(hipMalloc(&m->Y, sizeof(float) * b * 8));
+  const int nPair = (B + 31) / 32;
+  const size_t chunks = (nPair + chunk_pairs(nPair) - 1) / chunk_pairs(nPair);
+  MCHK(hipMalloc(&m->ops, sizeof(bf16x4) * 2 * nPair * NTB * 64));
+  MCHK(hipMalloc(&m->X, sizeof(float) * b * 16));
   MCHK(hipMalloc(&m->T, sizeof(float) * b * 8));
   MCHK(hipMalloc(&m->rowErr, sizeof(float) * b));
-  MCHK(hipMalloc(&m->rowW, sizeof(float) * b));
-  m->nSplit = (B + kChunkRows - 1) / kChunkRows;
-  MCHK(hipMalloc(&m->partial, sizeof(float) * (size_t)m->nSplit * NPARAM));
+  // (a smaller batch may take more, smaller chunks: up to 256)
+  MCHK(hipMalloc(&m->partial,
+                 sizeof(float) * (chunks > 256 ? chunks : 256) * NPARAM));
   m->cap = B;
   return BATS_OK;
 }
 
-static GemmArgs gemm0() {
-  GemmArgs g;
-  memset(&g, 0, sizeof g);
-  return g;
-}
-
-static void launch_gemm(int epi, const GemmArgs &g, hipStream_t s, int splits) {
-  const int tiles = ((g.M + 15) / 16) * ((g.N + 15) / 16);
-  const dim3 grid((tiles + 3) / 4, splits), blk(256);
-  switch (epi) {
-  case EPI_FWD: hipLaunchKernelGGL(k_gemm<EPI_FWD>, grid, blk, 0, s, g); break;
-  case EPI_OUT: hipLaunchKernelGGL(k_gemm<EPI_OUT>, grid, blk, 0, s, g); break;
-  case EPI_BWD: hipLaunchKernelGGL(k_gemm<EPI_BWD>, grid, blk, 0, s, g); break;
-  default: hipLaunchKernelGGL(k_gemm<EPI_WGRAD>, grid, blk, 0, s, g); break;
-  }
-}
-
-// forward of the minibatch in m->X (B rows) into Z1..Z3, A1..A3, Y
-static void forward_batch(bats_mlp *m, int B) {
-  const __bf16 *in[4] = {m->X, m->A1, m->A2, m->A3};
-  float *Z[4] = {m->Z1, m->Z2, m->Z3, m->Y};
-  __bf16 *Aout[3] = {m->A1, m->A2, m->A3};
-  for (int l = 0; l < NL; l++) {
-    GemmArgs g = gemm0();
-    g.M = B; g.N = DIM[l + 1]; g.K = DIM[l];
-    g.A = in[l]; g.sAm = DIM[l]; g.sAk = 1;
-    g.B = m->wb + OW[l]; g.sBk = DIM[l + 1]; g.sBn = 1;
-    g.bias = m->w + OB[l];
-    g.Cf = Z[l]; g.ldc = DIM[l + 1];
-    if (l < NL - 1) {
-      g.Cb = Aout[l];
-      launch_gemm(EPI_FWD, g, m->stream, 1);
-    } else {
-      launch_gemm(EPI_OUT, g, m->stream, 1);
-    }
-  }
-}
-
-// gradient of the mean-square loss of the minibatch (X, T already on the
-// device) into m->grad and, if lr > 0, one Adam step; rowErr filled
-// the step counter of graph-captured training, advanced after each step
-__global__ void k_step_inc(long *step) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *step += 1;
-}
-
-static int grad_step(bats_mlp *m, int B, float lr, bool update,
-                     const float *W = nullptr, const float *sched = nullptr,
-                     const long *dStep = nullptr) {
-  forward_batch(m, B);
-  hipLaunchKernelGGL(k_loss, dim3((B + 255) / 256), dim3(256), 0, m->stream,
-                     m->Y, m->T, W, B, m->dY, m->rowErr);
-  const __bf16 *Ain[4] = {m->X, m->A1, m->A2, m->A3};
-  __bf16 *dZ[4] = {m->dZ1, m->dZ2, m->dZ3, m->dY};
-  const float *Zs[3] = {m->Z1, m->Z2, m->Z3};
-  const int S = (B + kChunkRows - 1) / kChunkRows;
-  for (int l = NL - 1; l >= 0; l--) {
-    // weight gradient partials: dW_l = A_{l-1}^T dZ_l over row chunks
-    GemmArgs g = gemm0();
-    g.M = DIM[l]; g.N = DIM[l + 1]; g.K = B;
-    g.A = Ain[l]; g.sAm = 1; g.sAk = DIM[l];
-    g.B = dZ[l]; g.sBk = DIM[l + 1]; g.sBn = 1;
-    g.Cf = m->partial + OW[l]; g.ldc = DIM[l + 1];
-    g.kChunk = kChunkRows; g.partialStride = NPARAM;
-    launch_gemm(EPI_WGRAD, g, m->stream, S);
-    hipLaunchKernelGGL(k_colsum, dim3(S), dim3(256), 0, m->stream, dZ[l], B,
-                       DIM[l + 1], kChunkRows, m->partial, (long)NPARAM, OB[l]);
-    if (l > 0) {
-      // dZ_{l-1} = (dZ_l W_l^T) * silu'(Z_{l-1})
-      GemmArgs d = gemm0();
-      d.M = B; d.N = DIM[l]; d.K = DIM[l + 1];
-      d.A = dZ[l]; d.sAm = DIM[l + 1]; d.sAk = 1;
-      d.B = m->wb + OW[l]; d.sBk = 1; d.sBn = DIM[l + 1];
-      d.Cb = dZ[l - 1]; d.ldc = DIM[l]; d.Zprev = Zs[l - 1];
-      launch_gemm(EPI_BWD, d, m->stream, 1);
-    }
-  }
-  hipLaunchKernelGGL(k_sum_partials, dim3((NPARAM + 255) / 256), dim3(256), 0,
-                     m->stream, m->partial, S, m->grad);
-  if (update) {
-    AdamArgs a;
-    a.grad = m->grad; a.w = m->w; a.m = m->m; a.v = m->v; a.wb = m->wb;
-    a.b1 = 0.9f; a.b2 = 0.999f; a.eps = 1e-8f;
-    a.sched = sched;
-    a.step = dStep;
-    if (!sched) {
-      m->step++;
-      a.lr = lr;
-      a.bc1 = 1.f - powf(a.b1, (float)m->step);
-      a.bc2 = 1.f - powf(a.b2, (float)m->step);
-    } else {
-      a.lr = a.bc1 = a.bc2 = 0.f;
-    }
-    hipLaunchKernelGGL(k_adam, dim3((NPARAM + 255) / 256), dim3(256), 0,
-                       m->stream, a);
-    m->fragStale = 1;
-  }
+// gradient of the mean-square loss of the minibatch a describes into m->grad
+// (and rowErr), and with a schedule one Adam step
+static int grad_step(bats_mlp *m, TrainArgs a, const float *sched) {
+  a.frag = m->frag;
+  a.bfrag = m->bfrag;
+  a.w = m->w;
+  a.ops = m->ops;
+  a.rowErr = m->rowErr;
+  const int nPair = (a.B + 31) / 32, per = chunk_pairs(nPair);
+  const int nChunk = (nPair + per - 1) / per;
+  const int nWg = (2 * nPair + kTrainWaves - 1) / kTrainWaves;
+  hipLaunchKernelGGL(k_train_rows, dim3(nWg < 256 ? nWg : 256),
+                     dim3(kTrainThreads), 0, m->stream, a);
+  hipLaunchKernelGGL(k_train_wgrad, dim3(nChunk), dim3(256), 0, m->stream,
+                     m->ops, nPair, per, m->partial, a.step);
+  UpdateArgs u;
+  u.partial = m->partial;
+  u.nChunk = nChunk;
+  u.grad = m->grad;
+  u.adam = sched != nullptr;
+  u.w = m->w; u.m = m->m; u.v = m->v;
+  u.frag = m->frag; u.bfrag = m->bfrag;
+  u.b1 = 0.9f; u.b2 = 0.999f; u.eps = 1e-8f;
+  u.sched = sched;
+  u.step = a.step;
+  hipLaunchKernelGGL(k_train_update,
+                     dim3((NPARAM + kUpdateParams - 1) / kUpdateParams),
+                     dim3(256), 0, m->stream, u);
   MCHK(hipGetLastError());
   return BATS_OK;
 }
-
 
 extern "C" int bats_mlp_loss_grad(bats_mlp *m, const float *X, const float *T,
                                   int B, double *Loss, float *grad) {
   if (!m || !X || !T || B <= 0) return BATS_EINVAL;
   int st = ensure_batch(m, B);
   if (st) return st;
-  std::vector<__bf16> xb((size_t)B * 16);
-  for (size_t t = 0; t < xb.size(); t++) xb[t] = (__bf16)X[t];
-  MCHK(hipMemcpyAsync(m->X, xb.data(), sizeof(__bf16) * xb.size(),
+  st = repack(m);
+  if (st) return st;
+  MCHK(hipMemcpyAsync(m->X, X, sizeof(float) * (size_t)B * 16,
                       hipMemcpyHostToDevice, m->stream));
   MCHK(hipMemcpyAsync(m->T, T, sizeof(float) * (size_t)B * 8,
                       hipMemcpyHostToDevice, m->stream));
-  MCHK(hipStreamSynchronize(m->stream));
-  st = grad_step(m, B, 0.f, false);
+  TrainArgs ta{};
+  ta.X = m->X;
+  ta.T = m->T;
+  ta.B = B;
+  st = grad_step(m, ta, nullptr);
   if (st) return st;
   std::vector<float> e(B);
   MCHK(hipMemcpyAsync(e.data(), m->rowErr, sizeof(float) * B,
@@ -802,9 +924,10 @@ extern "C" int bats_mlp_train(bats_mlp *m, int nEpoch, int Batch, double Lr0,
                         m->stream));
     hipLaunchKernelGGL(k_scale_last, dim3(1), dim3(64 * 8 + 8), 0, m->stream,
                        m->w, dScale, 1);
-    hipLaunchKernelGGL(k_to_bf16, dim3((NPARAM + 255) / 256), dim3(256), 0,
-                       m->stream, m->w, m->wb, (long)NPARAM);
+    m->fragStale = 1;
   }
+  st = repack(m);
+  if (st) return st;
   // jump weights: each sample's squared error weighted by its jump norm
   // over the mean jump norm of the training samples
   float invMeanJ = 1.0f;
@@ -837,20 +960,22 @@ extern "C" int bats_mlp_train(bats_mlp *m, int nEpoch, int Batch, double Lr0,
     float *dSched = nullptr;
     long *dStep = nullptr;
     MCHK(hipMalloc(&dSched, sizeof(float) * sched.size()));
-    MCHK(hipMalloc(&dStep, sizeof(long)));
+    MCHK(hipMalloc(&dStep, 2 * sizeof(long)));
     MCHK(hipMemcpyAsync(dSched, sched.data(), sizeof(float) * sched.size(),
                         hipMemcpyHostToDevice, m->stream));
-    MCHK(hipMemsetAsync(dStep, 0, sizeof(long), m->stream));
-    float *W = JumpWeight ? m->rowW : nullptr;
+    MCHK(hipMemsetAsync(dStep, 0, 2 * sizeof(long), m->stream));
     // one training step: the same kernels whether captured or launched
-    auto one_step = [&]() {
-      hipLaunchKernelGGL(k_gather_rows, dim3((B + 255) / 256), dim3(256), 0,
-                         m->stream, m->dataX, m->dataT, dIdx, B, m->X, m->T,
-                         dScale, m->dataJ, invMeanJ, W, dStep, stepsPerEpoch);
-      const int r = grad_step(m, B, 0.f, true, W, dSched, dStep);
-      hipLaunchKernelGGL(k_step_inc, dim3(1), dim3(64), 0, m->stream, dStep);
-      return r;
-    };
+    TrainArgs ta{};
+    ta.X = m->dataX;
+    ta.T = m->dataT;
+    ta.J = JumpWeight ? m->dataJ : nullptr;
+    ta.invMeanJ = invMeanJ;
+    ta.scale = dScale;
+    ta.idx = dIdx;
+    ta.perEpoch = stepsPerEpoch;
+    ta.step = dStep;
+    ta.B = B;
+    auto one_step = [&]() { return grad_step(m, ta, dSched); };
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     if (UseGraph) {
@@ -878,7 +1003,8 @@ extern "C" int bats_mlp_train(bats_mlp *m, int nEpoch, int Batch, double Lr0,
           st = one_step();
       }
       if (st != BATS_OK) break;
-      // loss of the epoch's last minibatch
+      if (ep + 1 < nEpoch) continue;
+      // loss of the last minibatch
       if (hipMemcpyAsync(e.data(), m->rowErr, sizeof(float) * B,
                          hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
           hipStreamSynchronize(m->stream) != hipSuccess) {
@@ -903,8 +1029,6 @@ extern "C" int bats_mlp_train(bats_mlp *m, int nEpoch, int Batch, double Lr0,
   // back to physical targets (a no-op scale of one without Standardize)
   hipLaunchKernelGGL(k_scale_last, dim3(1), dim3(64 * 8 + 8), 0, m->stream,
                      m->w, dScale, 0);
-  hipLaunchKernelGGL(k_to_bf16, dim3((NPARAM + 255) / 256), dim3(256), 0,
-                     m->stream, m->w, m->wb, (long)NPARAM);
   m->fragStale = 1;
   MCHK(hipStreamSynchronize(m->stream));
   (void)hipFree(dScale);

@@ -17,6 +17,7 @@ namespace bats {
 namespace mlp {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 constexpr int NL = 4;                       // layers
@@ -53,6 +54,34 @@ constexpr int NFRAG = NTILE * TILE;         // 29696 bf16 = 58 KiB
 __host__ __device__ inline int frag_k(int layer, int kb, int g, int t) {
   if (layer == 0) return kb * 32 + 8 * g + t;
   return 32 * kb + (t < 4 ? 4 * g + t : 16 + 4 * g + (t - 4));
+}
+// the slot (g, t) of input k within its block of 32, the inverse of frag_k
+__host__ __device__ inline void frag_slot(int layer, int k, int &g, int &t) {
+  const int r = k % 32;
+  if (layer == 0) { g = r / 8; t = r % 8; }
+  else if (r < 16) { g = r / 4; t = r % 4; }
+  else { g = (r - 16) / 4; t = 4 + (r - 16) % 4; }
+}
+// the same for the way back: dA^T = W dZ^T of layers 2..4 takes W itself as
+// the A operand (16 inputs x 32 outputs per tile, tiles input block major),
+// the outputs in the order in which the layer's accumulators hold them
+constexpr int BT1 = 0, BT2 = BT1 + (128 / 16) * (128 / 32);
+constexpr int BT3 = BT2 + (128 / 16) * (64 / 32);
+constexpr int NBTILE = BT3 + 64 / 16;       // 52
+constexpr int BT[NL] = {0, BT1, BT2, BT3};
+constexpr int NBFRAG = NBTILE * TILE;       // 26624 bf16 = 52 KiB
+// position of parameter W_l[k][n] in the forward and the backward fragments
+__host__ __device__ inline int frag_pos(int l, int k, int n) {
+  int g, t;
+  frag_slot(l, k, g, t);
+  return ((FT[l] + (n / 16) * (KP[l] / 32) + k / 32) * 64 + 16 * g + n % 16) *
+             8 + t;
+}
+__host__ __device__ inline int bfrag_pos(int l, int k, int n) {
+  int g, t;
+  frag_slot(1, n, g, t);
+  const int nKb = l == 3 ? 1 : DIM[l + 1] / 32;
+  return ((BT[l] + (k / 16) * nKb + n / 32) * 64 + 16 * g + k % 16) * 8 + t;
 }
 // the biases packed for the inference kernel's LDS copy
 constexpr int CB1 = 0, CB2 = 128, CB3 = 256, CB4 = 320, NBIAS = 328;
