@@ -568,8 +568,7 @@ k_global_dt(const double *dtmaxB, const int *runFirst, double *scalAll,
   }
 }
 
-// fill n doubles with v (a kernel rather than a memset, so that a captured
-// step graph holds no memset node)
+// fill n doubles with v
 __global__ void __launch_bounds__(256) k_fill(double *p, long n, double v) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < n) p[t] = v;
@@ -704,6 +703,8 @@ extern "C" int bats_init(const bats_config *cfg, bats_handle **out) {
   if (e == hipSuccess) e = hipMalloc(&h->nei, sizeof(int) * 6 * c.nBlock);
   if (e == hipSuccess) e = hipMalloc(&h->cellsize, sizeof(double) * 3 * c.nBlock);
   if (e == hipSuccess) e = hipMalloc(&h->dtmaxB, sizeof(double) * c.nBlock);
+  if (e == hipSuccess) e = hipMalloc(&h->dtAcc, sizeof(*h->dtAcc) * c.nBlock);
+  if (e == hipSuccess) e = hipMalloc(&h->dtCnt, sizeof(*h->dtCnt) * c.nBlock);
   if (e == hipSuccess) e = hipMalloc(&h->scal, sizeof(double) * S_NSCAL);
   if (e == hipSuccess) e = hipMalloc(&h->runFirst, sizeof(int) * 2);
   if (e == hipSuccess) e = hipMalloc(&h->runOfBlock, sizeof(int) * c.nBlock);
@@ -738,6 +739,12 @@ extern "C" int bats_init(const bats_config *cfg, bats_handle **out) {
   HIPCHK(hipMemset(h->runOfBlock, 0, sizeof(int) * c.nBlock));
   HIPCHK(hipMemset(h->err, 0, sizeof(int)));
   HIPCHK(hipMemset(h->dtmaxB, 0, sizeof(double) * c.nBlock));
+  HIPCHK(hipMemset(h->dtCnt, 0, sizeof(*h->dtCnt) * c.nBlock));
+  hipLaunchKernelGGL(k_fill, dim3((c.nBlock + 255) / 256), dim3(256), 0,
+                     h->stream, reinterpret_cast<double *>(h->dtAcc),
+                     (long)c.nBlock, 1.7976931348623157e308);
+  HIPCHK(hipGetLastError());
+  h->splitShift = -1;
   // outer boundaries float until bats_set_cell_boundary
   for (int side = 0; side < 6; side++) h->bcType[side] = BATS_BC_FLOAT;
   HIPCHK(hipMalloc(&h->dBcState, sizeof h->bcState));
@@ -762,7 +769,7 @@ extern "C" int bats_finalize(bats_handle *h) {
   if (!h) return BATS_EINVAL;
   (void)hipStreamSynchronize(h->stream);
   void *ptrs[] = {h->U[0], h->U[1], h->U[2], h->Usnap, h->nei, h->cellsize, h->dtmaxB,
-                  h->dtmaxCB, h->scal, h->runFirst, h->runOfBlock, h->err,
+                  h->dtmaxCB, h->dtAcc, h->dtCnt, h->scal, h->runFirst, h->runOfBlock, h->err,
                   h->partial, h->LX, h->RX,
                   h->LY, h->RY, h->LZ, h->RZ, h->FX, h->FY, h->FZ, h->Src,
                   h->sur.face, h->sur.rowX, h->sur.rowFace, h->sur.rowScale,
@@ -1333,6 +1340,40 @@ extern "C" int bats_set_global_timestep(bats_handle *h, double TimeSimulationLim
   return BATS_OK;
 }
 
+// Parts (2^shift) into which the blocks' planes are cut when the caller sets
+// no launch shape.  A workgroup marches through its planes one behind the
+// other, about 8 us each, whatever else runs: a grid of few blocks is done
+// sooner in shorter parts, until all the places of the chip are taken (two
+// workgroups per CU in FP64, three in FP32), and a grid of a few times the
+// places ends with a nearly empty last round that shorter parts fill.  Each
+// part loads three planes more for its first face, about half a plane's
+// time.  The rule takes the least of rounds * (planes + 1/2); a last round
+// with at most one workgroup per CU takes 0.73 of a full one (FP32: 0.68,
+// with two 0.83), and beyond three rounds the workgroups no longer start
+// together, so that only the tail of the last one shows.  Measured, whole
+// blocks against the rule's parts (HLLD, per launch): FP64 8^3, 8 blocks 79
+// -> 20 us, 512 blocks 82 -> 38; 16^3, 64 blocks 143 -> 37, 105 blocks 141
+// -> 57, 256 blocks 140 -> 98, 600 blocks 336 -> 246; 512, 1000 and 4096
+// blocks stay whole (184, 381 us and 1.5 ms; in halves 186, 386 us).
+static int auto_split(int nGroup, int NB, bool f32) {
+  const int slots = f32 ? 768 : 512;
+  int best = 0;
+  double least = 0.0;
+  for (int s = 0; (NB >> s) >= 1; s++) {
+    const long items = (long)nGroup << s;
+    const long q = items / slots, rem = items % slots;
+    double rounds = (double)q;
+    if (q >= 3)
+      rounds = (double)items / slots + 0.15;
+    else if (rem > 0)
+      rounds += f32 ? (rem <= 256 ? 0.68 : rem <= 512 ? 0.83 : 1.0)
+                    : (rem <= 256 ? 0.73 : 1.0);
+    const double cost = rounds * ((NB >> s) + 0.5);
+    if (s == 0 || cost < least) { least = cost; best = s; }
+  }
+  return best;
+}
+
 // calcDt: DoCalcTimestep of the stage loop.  The local time steps are set
 // after the last stage's update (time accurate, :217-219), before the first
 // stage's update (steady state, :184-195), and always by the no-update pass.
@@ -1386,7 +1427,13 @@ static int launch_stage(bats_handle *h, int iStage, int calcDt, int noUpdate,
   a.advanceTime = advanceTime && !steady;
   const int NB = h->NB;
   a.nGroup = (c.nBlock + kThreads / (NB * NB) - 1) / (kThreads / (NB * NB));
-  a.splitShift = h->splitShift;
+  // a persistent grid walks whole blocks
+  const bool autoShape = h->splitShift < 0 && h->nWorkgroupMax == 0;
+  const bool f32 = h->elemSize == 4;
+  a.splitShift = autoShape ? auto_split(a.nGroup, NB, f32)
+                           : std::max(h->splitShift, 0);
+  a.dtAcc = h->dtAcc;
+  a.dtCnt = h->dtCnt;
   a.xcdOrder = h->xcdOrder;
   a.nWorkgroup = h->nWorkgroupMax > 0 ? h->nWorkgroupMax
                                       : a.nGroup << a.splitShift;
@@ -1428,7 +1475,6 @@ static int launch_stage(bats_handle *h, int iStage, int calcDt, int noUpdate,
   a.b0C = h->b0C;
   a.useB0Src = h->useB0Src;
   a.steady = steady;
-  const bool f32 = h->elemSize == 4;
   hipError_t e = hipSuccess;
   // resolution changes: ghost slabs of the stage input
   if (h->nSlab > 0) {
@@ -1485,17 +1531,17 @@ static int launch_stage(bats_handle *h, int iStage, int calcDt, int noUpdate,
     if (st) return st;
   } else {
     // the few groups with a body block would leave most of the GPU idle in
-    // their own launch: their blocks are cut into z-parts of at least two
-    // planes until about one workgroup per CU runs
+    // their own launch: their blocks are cut by the same rule, or with a
+    // given shape into z-parts of at least two planes until about one
+    // workgroup per CU runs
     int bodyShift = a.splitShift;
-    if (h->useBody)
+    if (h->useBody && autoShape) {
+      bodyShift = auto_split(h->nBodyGroup, NB, f32);
+      if (h->nPlainGroup > 0)
+        a.splitShift = auto_split(h->nPlainGroup, NB, f32);
+    } else if (h->useBody) {
       while ((h->nBodyGroup << bodyShift) < 256 && (NB >> (bodyShift + 1)) >= 2)
         bodyShift++;
-    // the parts of a split block meet in an atomic minimum of dtmaxB
-    if (a.doDt && (a.splitShift || bodyShift)) {
-      const long n = c.nBlock;
-      hipLaunchKernelGGL(k_fill, dim3((unsigned)((n + 255) / 256)), dim3(256),
-                         0, h->stream, h->dtmaxB, n, 1.7976931348623157e308);
     }
     auto launch = [&](const StageArgs &la, int lopt) {
 #define BATS_PICK(NBv, FL)                                                   \

@@ -55,7 +55,10 @@ struct bats_handle {
   int *runOfBlock;   // nBlock
   int nWorkgroupMax; // > 0: persistent grid of at most this many workgroups
   int splitShift;    // each block's planes split over 2^splitShift work
-                     // items (cells per thread NB >> splitShift)
+                     // items (cells per thread NB >> splitShift); -1: chosen
+                     // by the number of blocks (auto_split)
+  unsigned long long *dtAcc;  // split blocks: the parts' time step minimum
+  unsigned *dtCnt;            // and count (StageArgs)
   int xcdOrder;      // XCD-contiguous order of the work items
   int *err;
   double *partial;

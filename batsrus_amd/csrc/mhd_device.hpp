@@ -254,9 +254,13 @@ __device__ __forceinline__ Real cell_beta(Real beta, Real betaRC, int nFace,
 }
 
 // conserved (p stored) -> primitive, u = (1/rho)*rho*u
-// (src/ModFaceValue.f90:1541,1581-1582)
+// (src/ModFaceValue.f90:1541,1581-1582); the velocities are rounded here
+// (no FMA with a difference that uses one of them once, as the first cell of
+// a z window is), so that a cell's slopes round the same wherever they are
+// formed
 template <typename Real>
 __device__ __forceinline__ void to_primitive(Real *q) {
+#pragma clang fp contract(off)
   const Real RhoInv = frcp(q[RHO]);
   q[MX] = RhoInv * q[MX];
   q[MY] = RhoInv * q[MY];

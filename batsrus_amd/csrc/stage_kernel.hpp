@@ -52,6 +52,10 @@ struct StageArgs {
   const int *runOfBlock;  // run index of each block (null: one run)
   int nRun;
   double *dtmaxB;      // per block minimum of the local time step
+  // split blocks: the minimum over the parts done so far (bit patterns,
+  // DBL_MAX between launches) and their number (0 between launches)
+  unsigned long long *dtAcc;
+  unsigned *dtCnt;
   double *dtmaxCB;     // optional per-cell local time step
   int *err;
   int nBlock;
@@ -609,12 +613,11 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
     };
 
     if (act) {
-      // prologue: slopes of cell k0-1 and the face below cell k0
+      // prologue: slopes of cell k0-1
       T Pm2[NVAR];
       load_prim(k0 - 2, Pm2);
       load_prim(k0 - 1, Q1);
       load_prim(k0, Q2);
-      load_prim(k0 + 1, Q3);
       const T bz = betaZ(k0 - 1);
 #pragma unroll
       for (int v = 0; v < NVAR; v++) {
@@ -622,24 +625,31 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
         slopes<LIM>(bz, Pm2[v], Q1[v], Q2[v], dl, dr);
         dLk[v] = dl;
       }
-      zface(FzLo, k0);
-      if (a.corr && k0 == 0) {
-        corrected(bb, 4, i, j, FzLo);
-        if (POWELL) corrected_bn(bb, 4, i, j, FzLo[NFZ - 2], FzLo[NFZ - 1]);
-      }
-#pragma unroll
-      for (int v = 0; v < NVAR; v++) { Q1[v] = Q2[v]; Q2[v] = Q3[v]; }
     }
 
-    for (int k = k0; k < k1; k++) {
+    // plane k0-1 gives only the z face below plane k0: one copy of the z
+    // face's code, so that a block split into parts rounds as a whole one
+    for (int k = k0 - 1; k < k1; k++) {
+      const bool first = k < k0;
       // z face k+1 of this column
       if (act) {
         load_prim(k + 2, Q3);
         zface(FzHi, k + 1);
-        if (a.corr && k == NB - 1) {
-          corrected(bb, 5, i, j, FzHi);
-          if (POWELL) corrected_bn(bb, 5, i, j, FzHi[NFZ - 2], FzHi[NFZ - 1]);
+        if (a.corr && (k == -1 || k == NB - 1)) {
+          const int side = first ? 4 : 5;
+          corrected(bb, side, i, j, FzHi);
+          if (POWELL)
+            corrected_bn(bb, side, i, j, FzHi[NFZ - 2], FzHi[NFZ - 1]);
         }
+      }
+      if (first) {
+#pragma unroll
+        for (int v = 0; v < NVAR; v++) { Q1[v] = Q2[v]; Q2[v] = Q3[v]; }
+#pragma unroll
+        for (int v = 0; v < NFZ; v++) FzLo[v] = FzHi[v];
+        continue;
+      }
+      if (act) {
         // own primitive of plane k
 #pragma unroll
         for (int v = 0; v < NVAR; v++) sP[sPi(lb, v, j + 2, i + 2)] = Q1[v];
@@ -1016,11 +1026,22 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
         double r = sRed[(lb * NC) / 64];
         for (int q = 1; q < WPB; q++) r = fmin2(r, sRed[(lb * NC) / 64 + q]);
         // the parts of a split block meet in an atomic minimum over the
-        // bit patterns (an order-preserving map for non-negative doubles;
-        // the launcher fills dtmaxB with DBL_MAX first)
-        if (a.splitShift)
-          atomicMin(reinterpret_cast<unsigned long long *>(a.dtmaxB + b),
-                    (unsigned long long)__double_as_longlong(r));
+        // bit patterns (an order-preserving map for non-negative doubles);
+        // the last one to come takes the result and leaves the two words
+        // as it found them.  The count is raised only after the minimum
+        // has returned, so the last part sees every other one's.
+        if (a.splitShift) {
+          const unsigned long long old =
+              atomicMin(a.dtAcc + b,
+                        (unsigned long long)__double_as_longlong(r));
+          asm volatile("" ::"v"(old) : "memory");
+          const unsigned last = (1u << a.splitShift) - 1;
+          if (atomicInc(a.dtCnt + b, last) == last)
+            a.dtmaxB[b] = __longlong_as_double((long long)atomicExch(
+                a.dtAcc + b,
+                (unsigned long long)__double_as_longlong(
+                    1.7976931348623157e308)));
+        }
         else
           a.dtmaxB[b] = r;
       }
