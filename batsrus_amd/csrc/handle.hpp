@@ -42,6 +42,10 @@ struct bats_handle {
   int stateBuf;  // buffer holding the current State_VGB (differs from cur
                  // between the stages of a 2-stage step)
   double *Usnap;
+  // pinned slots of the host threads that move a large state in or out, and
+  // the events of the copies through them (made on first use)
+  void *slotMem;
+  hipEvent_t slotEv[8];
   void *lowCrit;  // low order face weights (elemSize-byte reals,
                   // 3*NB^2*(NB+1) per block, crit_index order) or null
   int *nei;
