@@ -21,10 +21,11 @@
 namespace bats {
 hipError_t BATS_NAME(BATS_NB, BATS_FLUX, BATS_REAL)(const StageArgs &a,
                                                     int opt,
-                                                    hipStream_t stream) {
+                                                    hipStream_t stream,
+                                                    LaunchEvents ev) {
   return launch_stage_kernel<BATS_NB, BATS_PASTE(BATS_FLUX_, BATS_FLUX),
-                             BATS_PASTE(BATS_REAL_, BATS_REAL)>(a, opt,
-                                                                stream);
+                             BATS_PASTE(BATS_REAL_, BATS_REAL)>(
+      a, opt, stream, ev);
 }
 #define BATS_FNAME_(nb, fl, ty) launch_fineflux_##nb##_##fl##_##ty
 #define BATS_FNAME(nb, fl, ty) BATS_FNAME_(nb, fl, ty)

@@ -28,6 +28,7 @@
 // The kernel is instantiated per (block size, flux) in its own translation
 // unit (stage_inst.hip) so the instantiations compile in parallel.
 #pragma once
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include "mhd_device.hpp"
@@ -1445,16 +1446,29 @@ inline hipError_t launch_amr_fineflux(const AmrArgs &a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Events that take the times of the kernel launched with them: its own start
+// and end, without the marker that an event recorded on the stream puts
+// between two kernels (null: not timed)
+struct LaunchEvents {
+  hipEvent_t start, stop;
+};
+
 // Launch k_stage for one block size and flux; the limiter and the options
 // (OPT_* bits) are dispatched here.
 template <int NB, int FLUX, typename T>
 inline hipError_t launch_stage_kernel(const StageArgs &a, int opt,
-                                      hipStream_t stream) {
+                                      hipStream_t stream, LaunchEvents ev) {
   const int nItem = a.nGroup << a.splitShift;
   const dim3 grid(nItem < a.nWorkgroup ? nItem : a.nWorkgroup),
       block(kThreads);
-#define BATS_K(LM, O)                                                        \
-  hipLaunchKernelGGL((k_stage<NB, FLUX, LM, O, T>), grid, block, 0, stream, a)
+  auto go = [&](void (*kernel)(StageArgs)) {
+    if (ev.start || ev.stop)
+      hipExtLaunchKernelGGL(kernel, grid, block, 0, stream, ev.start, ev.stop,
+                            0, a);
+    else
+      hipLaunchKernelGGL(kernel, grid, block, 0, stream, a);
+  };
+#define BATS_K(LM, O) go(k_stage<NB, FLUX, LM, O, T>)
   // the limiters without beta never take OPT_RESBETA (no instances)
 #define BATS_LAUNCH3(LM)                                                     \
   switch (opt & 11) {                                                        \
@@ -1623,7 +1637,7 @@ inline hipError_t launch_stage_kernel(const StageArgs &a, int opt,
 // (stage_inst.hip)
 #define BATS_DECLARE_LAUNCH(NB, FL, TY)                                     \
   hipError_t launch_stage_##NB##_##FL##_##TY(const StageArgs &, int,        \
-                                             hipStream_t);
+                                             hipStream_t, LaunchEvents);
 #define BATS_DECLARE_LAUNCH_FLUX(NB, TY)                                    \
   BATS_DECLARE_LAUNCH(NB, rusanov, TY)                                      \
   BATS_DECLARE_LAUNCH(NB, linde, TY)                                        \
