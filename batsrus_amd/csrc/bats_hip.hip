@@ -775,8 +775,7 @@ extern "C" int bats_finalize(bats_handle *h) {
                   h->dtmaxCB, h->dtAcc, h->dtCnt, h->scal, h->runFirst, h->runOfBlock, h->err,
                   h->partial, h->LX, h->RX,
                   h->LY, h->RY, h->LZ, h->RZ, h->FX, h->FY, h->FZ, h->Src,
-                  h->sur.face, h->sur.rowX, h->sur.rowFace, h->sur.rowScale,
-                  h->sur.counters, h->slabs, h->slabKind, h->fineSlabs,
+                  h->sur.face, h->sur.counters, h->slabs, h->slabKind, h->fineSlabs,
                   h->corr, h->lowCrit, h->dBcState, h->b0F, h->b0C,
                   h->bodySlot, h->bodyUsed, h->bodyXyz0, h->groupList,
                   h->b0Side, h->b0SideSlot, h->varyT, h->varyS};

@@ -18,11 +18,6 @@ struct SurrogateState {
   double betaMin;      // gate: minimum plasma beta for the network
   double jumpTol;      // gate: largest scaled jump counted as smooth
   float *face;         // face fluxes, 9 slots per face, all blocks
-  __bf16 *rowX;        // network inputs of the gated faces (rows x 16)
-  float *rowY;         // network outputs (rows x 8)
-  int *rowFace;        // per row: global face index
-  float *rowScale;     // per row (float4): density scale, speed scale,
-                       // jump norm, face area
   int *counters;       // [0] rows this stage; 64-bit at [2] faces and at
                        // [4] network rows since set_surrogate
   long faceCap;

@@ -431,7 +431,7 @@ __global__ void k_pack_frag(const float *w, __bf16 *frag, __bf16 *bfrag) {
 
 namespace {
 
-__global__ void __launch_bounds__(kInferThreads, 8)
+__global__ void __launch_bounds__(kInferThreads, 4)
 k_infer(const __bf16 *frag, const float *w, const float *X, float *Y,
         int rows) {
   __shared__ __attribute__((aligned(16))) __bf16 sW[NFRAG];
@@ -440,12 +440,25 @@ k_infer(const __bf16 *frag, const float *w, const float *X, float *Y,
     reinterpret_cast<bf16x8 *>(sW)[t] = reinterpret_cast<const bf16x8 *>(frag)[t];
   load_biases(w, sBias);
   __syncthreads();
-  const int wave = threadIdx.x >> 6;
-  const int nTile = (rows + 15) / 16;
-  auto out = [&](int row, int col, float v) { Y[(long)row * 8 + col] = v; };
-  for (int tile = blockIdx.x * kInferWaves + wave; tile < nTile;
-       tile += gridDim.x * kInferWaves)
-    infer_tile(sW, sBias, X, rows, tile * 16, out);
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int nPair = (rows + 31) / 32;
+  for (int pair = blockIdx.x * kInferWaves + (threadIdx.x >> 6); pair < nPair;
+       pair += gridDim.x * kInferWaves) {
+    bf16x8 x[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const int row = pair * 32 + 16 * h + r;
+#pragma unroll
+      for (int t = 0; t < 8; t++)
+        x[h][t] = (g < 2 && row < rows)
+                      ? (__bf16)X[(long)row * 16 + 8 * g + t] : (__bf16)0.f;
+    }
+    infer_tiles<2>(sW, sBias, x, [&](int h, f32x4 y) {
+      const int row = pair * 32 + 16 * h + r;
+      if (g < 2 && row < rows)
+        *reinterpret_cast<f32x4 *>(Y + (long)row * 8 + 4 * g) = y;
+    });
+  }
 }
 
 __global__ void k_gather_rows_f32(const float *dataX, const float *dataT,
@@ -749,8 +762,8 @@ int bats::mlp::forward_device(bats_mlp *m, const float *dX, float *dY,
   int st = repack(m);
   if (st) return st;
   MCHK(hipStreamSynchronize(m->stream));
-  const int nTile = (rows + 15) / 16;
-  int grid = (nTile + kInferWaves - 1) / kInferWaves;
+  const int nPair = (rows + 31) / 32;
+  int grid = (nPair + kInferWaves - 1) / kInferWaves;
   if (grid > kInferGrid) grid = kInferGrid;
   hipLaunchKernelGGL(k_infer, dim3(grid), dim3(kInferThreads), 0, stream, m->frag, m->w,
                      dX, dY, rows);

@@ -13,6 +13,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace bats {
 namespace mlp {
 
@@ -116,98 +118,84 @@ __device__ __forceinline__ float dsilu(float z) {
 // batched inference: Y[rows x 8] = MLP(X[rows x 16]) with fragment-ordered
 // BF16 weights (flat FP32 biases); a workgroup walks 64-row groups
 // =====================================================================
-// inference workgroups: 16 waves share one LDS copy of the weights (59 KiB);
-// two workgroups per CU, 8 waves per SIMD (at most 64 VGPRs)
-constexpr int kInferThreads = 1024, kInferWaves = kInferThreads / 64;
+// inference workgroups: 8 waves share one LDS copy of the weights (59 KiB);
+// two workgroups per CU, 4 waves per SIMD (at most 128 VGPRs)
+constexpr int kInferThreads = 512, kInferWaves = kInferThreads / 64;
 constexpr int kInferGrid = 2 * 256;
 
-// one 16-row tile through the network; X rows are FP32, Y rows FP32.  sW:
-// fragments in LDS, bias: the packed biases (load_biases) in LDS.  The
-// activations never leave the registers: each layer's accumulators, through
-// SiLU and BF16, are the next layer's B fragments (see frag_k).
-// X rows are FP32 (rounded to BF16 here) or already BF16.
-template <typename XT, typename OUT>
-__device__ __forceinline__ void infer_tile(const __bf16 *sW, const float *bias,
-                                           const XT *X, int rows, int r0,
-                                           OUT out) {
-  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const bf16x8 *W = reinterpret_cast<const bf16x8 *>(sW);
-  // layer 1: B fragment straight from X (inputs k >= 16 are padding)
-  bf16x8 x;
-  const int row0 = r0 + r;
-  if (sizeof(XT) == 2) {
-    // 16-byte load of inputs 8g .. 8g+7 of the row
-    x = (g < 2 && row0 < rows)
-            ? *reinterpret_cast<const bf16x8 *>(X + (long)row0 * 16 + 8 * g)
-            : bf16x8{};
-  } else {
-#pragma unroll
-    for (int t = 0; t < 8; t++) {
-      const int k = 8 * g + t;
-      x[t] = (k < 16 && row0 < rows) ? (__bf16)X[(long)row0 * 16 + k]
-                                     : (__bf16)0.f;
-    }
-  }
+// R tiles of 16 rows through the network, x[t] the input fragment of tile t
+// (lane l: inputs 8 (l/16) .. +7 of row l%16, zero from input 16 on).  sW:
+// weight fragments in LDS, bias: the packed biases (load_biases) in LDS.  The
+// activations never leave the registers: two output blocks of a layer,
+// through SiLU and BF16, are one B fragment of the next (see frag_k), formed
+// while the matrix cores work on the following two.  A weight fragment is
+// read from LDS once for all R tiles.  out(t, y): lanes with l/16 < 2 hold
+// outputs 4 (l/16) .. +3 of row l%16 of tile t.
+template <int R, typename OUT>
+__device__ __forceinline__ void infer_tiles(const __bf16 *sW,
+                                            const float *bias,
+                                            const bf16x8 (&x)[R], OUT out) {
+  const int lane = threadIdx.x & 63, g = lane >> 4;
+  const bf16x8 *W = reinterpret_cast<const bf16x8 *>(sW) + lane;
   // accumulators start at the bias of their outputs 16 nb + 4 g + i
   auto bias4 = [&](const float *b, int nb) {
     const float *p = b + nb * 16 + 4 * g;
     return f32x4{p[0], p[1], p[2], p[3]};
   };
-  // SiLU of output blocks 2 kb and 2 kb + 1 -> B fragment kb
-  auto act = [&](const f32x4 *a, int kb) {
-    bf16x8 v;
+  // one layer: NK input fragments to NO output fragments per tile
+  auto layer = [&](auto nk, auto no, int ft, const float *b,
+                   const auto &in, auto &o) {
+    constexpr int NK = decltype(nk)::value, NO = decltype(no)::value;
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-      v[t] = (__bf16)silu(a[2 * kb][t]);
-      v[4 + t] = (__bf16)silu(a[2 * kb + 1][t]);
-    }
-    return v;
-  };
-  f32x4 acc[8];
+    for (int kb = 0; kb < NO; kb++) {
+      f32x4 acc[R][2];
 #pragma unroll
-  for (int nb = 0; nb < 8; nb++) {
-    acc[nb] = mfma(W[(FT0 + nb) * 64 + lane], x, bias4(bias + CB1, nb));
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  bf16x8 b4[4];
+      for (int h = 0; h < 2; h++) {
+        const int nb = 2 * kb + h;
+        const f32x4 b4 = bias4(b, nb);
 #pragma unroll
-  for (int kb = 0; kb < 4; kb++) b4[kb] = act(acc, kb);
-  // layer 2: 128 -> 128
+        for (int t = 0; t < R; t++) acc[t][h] = b4;
 #pragma unroll
-  for (int nb = 0; nb < 8; nb++) {
-    acc[nb] = bias4(bias + CB2, nb);
+        for (int q = 0; q < NK; q++) {
+          const bf16x8 w = W[(ft + nb * NK + q) * 64];
 #pragma unroll
-    for (int kb = 0; kb < 4; kb++)
-      acc[nb] = mfma(W[(FT1 + nb * 4 + kb) * 64 + lane], b4[kb], acc[nb]);
-    // keep the weight fragments of one output block live at a time
-    __builtin_amdgcn_sched_barrier(0);
-  }
-#pragma unroll
-  for (int kb = 0; kb < 4; kb++) b4[kb] = act(acc, kb);
-  // layer 3: 128 -> 64
-#pragma unroll
-  for (int nb = 0; nb < 4; nb++) {
-    acc[nb] = bias4(bias + CB3, nb);
-#pragma unroll
-    for (int kb = 0; kb < 4; kb++)
-      acc[nb] = mfma(W[(FT2 + nb * 4 + kb) * 64 + lane], b4[kb], acc[nb]);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-#pragma unroll
-  for (int kb = 0; kb < 2; kb++) b4[kb] = act(acc, kb);
-  // layer 4: 64 -> 8 (padded to 16 outputs; lanes with g < 2 hold 0..7)
-  f32x4 y = {0.f, 0.f, 0.f, 0.f};
-  y = mfma(W[(FT3 + 0) * 64 + lane], b4[0], y);
-  y = mfma(W[(FT3 + 1) * 64 + lane], b4[1], y);
-  if (g < 2) {
-    const int row = r0 + r;
-    if (row < rows) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int n = 4 * g + i;
-        out(row, n, y[i] + bias[CB4 + n]);
+          for (int t = 0; t < R; t++) acc[t][h] = mfma(w, in[t][q], acc[t][h]);
+        }
       }
+#pragma unroll
+      for (int t = 0; t < R; t++) {
+        bf16x8 v;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          v[i] = (__bf16)silu(acc[t][0][i]);
+          v[4 + i] = (__bf16)silu(acc[t][1][i]);
+        }
+        o[t][kb] = v;
+      }
+      // the weight fragments of two output blocks live at a time
+      __builtin_amdgcn_sched_barrier(0);
     }
+  };
+  using std::integral_constant;
+  bf16x8 f0[R][1], f1[R][4], f2[R][4], f3[R][2];
+#pragma unroll
+  for (int t = 0; t < R; t++) f0[t][0] = x[t];
+  layer(integral_constant<int, 1>(), integral_constant<int, 4>(), FT0,
+        bias + CB1, f0, f1);
+  layer(integral_constant<int, 4>(), integral_constant<int, 4>(), FT1,
+        bias + CB2, f1, f2);
+  layer(integral_constant<int, 4>(), integral_constant<int, 2>(), FT2,
+        bias + CB3, f2, f3);
+  // layer 4: 64 -> 8 (padded to 16 outputs)
+#pragma unroll
+  for (int t = 0; t < R; t++) {
+    f32x4 y = {0.f, 0.f, 0.f, 0.f};
+    y = mfma(W[(FT3 + 0) * 64], f3[t][0], y);
+    y = mfma(W[(FT3 + 1) * 64], f3[t][1], y);
+    const float *p = bias + CB4 + 4 * (g & 1);
+#pragma unroll
+    for (int i = 0; i < 4; i++) y[i] += p[i];
+    out(t, y);
   }
 }
 

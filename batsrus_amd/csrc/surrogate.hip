@@ -31,13 +31,13 @@
 // BetaMin.  Every other face takes the exact flux.
 //
 // Surrogate stage (FP32 state):
-//   k_sur_faces   face states, gate, Vdt; exact flux of the gated-out faces
-//                 into the face array; compacted network input rows
-//   k_sur_infer   the network on the rows (matrix cores), fluxes scattered
-//                 back to the face array in the original frame, times area
+//   k_sur_faces   face states, gate, Vdt; the exact flux of the gated-out
+//                 faces, the Rusanov flux plus the network's correction of
+//                 the others (matrix cores), into the face array
 //   k_sur_update  flux divergence, stage update in FP64, local time step
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -317,35 +317,58 @@ struct SurArgs {
       noUpdate, advanceTime;
   float *face;     // NSLOT x nFaceTot
   long nFaceTot;   // 3 * nBlock * NF
-  __bf16 *rowX;
-  int *rowFace;
-  float *rowScale;
+  const __bf16 *frag;  // the network's weights (network mode)
+  const float *w;
   int *counters;
 };
 
-template <int NB, int LIM>
-__global__ void __launch_bounds__(256) k_sur_faces(SurArgs a) {
+// faces of a workgroup's round: network mode keeps the weights in LDS (75
+// KiB with the rows on their way, two workgroups per CU, four waves per SIMD)
+constexpr int kNetThreads = 512;
+
+// One face per lane.  NET: a wave packs the inputs of its faces that passed
+// the gate into rows in LDS, takes them through the network 32 at a time and
+// adds each correction to the flux its lane still holds, so a face's flux is
+// written once and no input, scale or index of it ever.  The two together
+// are bound by the vector unit (SiLU's two transcendentals per activation);
+// apart, the rows cost 204 bytes of memory traffic per face: 722 + 328 us per
+// stage at 6.7 million faces, 818 us now.
+template <int NB, int LIM, bool NET>
+__global__ void __launch_bounds__(NET ? kNetThreads : 256, NET ? 4 : 1)
+k_sur_faces(SurArgs a) {
   using G = FaceGeom<NB>;
+  using namespace bats::mlp;
+  __shared__ __attribute__((aligned(16))) __bf16 sW[NET ? NFRAG : 8];
+  __shared__ float sBias[NET ? NBIAS : 1];
+  // per wave: 64 rows of 16 inputs (BF16), then of 8 outputs (FP32)
+  __shared__ __attribute__((aligned(16))) __bf16
+      sRow[NET ? (kNetThreads / 64) * 64 * 16 : 8];
+  if (NET) {
+    for (int t = threadIdx.x; t < NFRAG / 8; t += kNetThreads)
+      reinterpret_cast<bf16x8 *>(sW)[t] =
+          reinterpret_cast<const bf16x8 *>(a.frag)[t];
+    load_biases(a.w, sBias);
+    __syncthreads();
+  }
+  const int lane = threadIdx.x & 63;
+  __bf16 *rows = sRow + (NET ? (threadIdx.x >> 6) * 64 * 16 : 0);
   const PhysT<float> ph = phys_as<float>(a.ph);
   const float beta = float(a.beta), betaMin = float(a.betaMin);
-  int err = 0;
-  long nNet = 0;
-  const long nTot = a.nFaceTot;
-  // per-wave row counts and the workgroup's base row, double-buffered by
-  // iteration so a wave can start the next iteration while another still
-  // reads this one's
-  __shared__ int sCountBuf[2][5];
-  int par = 0;
-  for (long gf = blockIdx.x * (long)blockDim.x + threadIdx.x;
-       gf - threadIdx.x < nTot; gf += (long)gridDim.x * blockDim.x, par ^= 1) {
-    int *sCount = sCountBuf[par];
+  int err = 0, nNet = 0;
+  // face indices fit 32 bits (bats_set_surrogate)
+  const unsigned nTot = (unsigned)a.nFaceTot;
+  const unsigned nDir = (unsigned)a.nBlock * G::NF;
+  for (unsigned w0 = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); w0 < nTot;
+       w0 += gridDim.x * blockDim.x) {
+    const unsigned gf = w0 + lane;
     const bool valid = gf < nTot;
     bool net = false;
     float x[16];
     float rhos = 0.f, cs = 0.f, jn = 0.f, area = 0.f;
+    float F[NFLUX];
+    const int dir = gf < nDir ? 0 : gf - nDir < nDir ? 1 : 2;
     if (valid) {
-      const int dir = (int)(gf / ((long)a.nBlock * G::NF));
-      const long rem = gf % ((long)a.nBlock * G::NF);
+      const unsigned rem = gf - dir * nDir;
       const int b = (int)(rem / G::NF), r = (int)(rem % G::NF);
       int fi, fj, fk;
       G::decode(dir, r, fi, fj, fk);
@@ -369,8 +392,8 @@ __global__ void __launch_bounds__(256) k_sur_faces(SurArgs a) {
       const bool smooth = ok && cs > 0.f &&
                           face_smooth(q[0], q[1], q[2], q[3], L, R, beta,
                                       betaMin, float(a.jumpTol), rhos, cs);
-      float F[NFLUX], vdt, unA;
-      if (smooth && a.mode == BATS_SUR_NETWORK) {
+      float vdt, unA;
+      if (NET && smooth) {
         // exact Vdt from the HLLD speeds; the flux comes from the network
         // HLLD's Cmax = max(sR, -sL) of the Linde-corrected states
         float Lc[NVAR], Rc[NVAR];
@@ -388,7 +411,6 @@ __global__ void __launch_bounds__(256) k_sur_faces(SurArgs a) {
         else if (dir == 1) err |= numerical_flux<1, FLUX_RUSANOV, false>(ph, area, L, R, F, vdt, unA);
         else err |= numerical_flux<2, FLUX_RUSANOV, false>(ph, area, L, R, F, vdt, unA);
         F[PP] = fmax2(sR, -sL) * area;
-        for (int v = 0; v < NSLOT; v++) a.face[v * nTot + gf] = F[v];
         net = jn > 0.f;  // no correction where the face states agree
       } else {
         if (smooth) {  // the method without the network: Rusanov
@@ -401,78 +423,81 @@ __global__ void __launch_bounds__(256) k_sur_faces(SurArgs a) {
           else err |= numerical_flux<2, FLUX_HLLD, false>(ph, area, L, R, F, vdt, unA);
         }
         F[PP] = vdt;
-        for (int v = 0; v < NSLOT; v++) a.face[v * nTot + gf] = F[v];
       }
     }
-    // workgroup-aggregated row allocation for the network faces: one
-    // atomic per workgroup and iteration (the loop trip count is uniform
-    // over the workgroup)
-    const unsigned long long mask = __ballot(net);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) sCount[wave] = __popcll(mask);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int tot = 0;
-      for (int w = 0; w < 4; w++) tot += sCount[w];
-      sCount[4] = tot ? atomicAdd(&a.counters[0], tot) : 0;
-    }
-    __syncthreads();
-    if (mask) {
-      int base = sCount[4];
-      for (int w = 0; w < wave; w++) base += sCount[w];
+    const unsigned long long mask = NET ? __ballot(net) : 0;
+    if (NET && mask) {
+      const int n = __popcll(mask), row = __popcll(mask & ((1ull << lane) - 1));
+      nNet += n;
+      // rows in and out of LDS belong to this wave alone: its LDS accesses
+      // happen in order, only the compiler has to keep it
+      auto order = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      };
+      bf16x8 *xr = reinterpret_cast<bf16x8 *>(rows);
       if (net) {
-        const int row = base + __popcll(mask & ((1ull << lane) - 1ull));
-        // the row's inputs in BF16 (the network's input precision; two
-        // 16-byte stores), then its scales
-        bats::mlp::bf16x8 x0, x1;
+        bf16x8 x0, x1;
 #pragma unroll
         for (int c = 0; c < 8; c++) {
           x0[c] = (__bf16)x[c];
           x1[c] = (__bf16)x[8 + c];
         }
-        bats::mlp::bf16x8 *xr =
-            reinterpret_cast<bats::mlp::bf16x8 *>(a.rowX + (long)row * 16);
-        xr[0] = x0;
-        xr[1] = x1;
-        a.rowFace[row] = (int)gf;
-        reinterpret_cast<float4 *>(a.rowScale)[row] =
-            make_float4(rhos, cs, jn, area);
+        xr[row * 2] = x0;
+        xr[row * 2 + 1] = x1;
       }
-      nNet += net ? 1 : 0;
+      order();
+      const int r = lane & 15, g = lane >> 4;
+      auto input = [&](int t0) {
+        return g < 2 && t0 + r < n ? xr[(t0 + r) * 2 + g] : bf16x8{};
+      };
+      // outputs over the inputs of rows that are through: 32 bytes each
+      float *yr = reinterpret_cast<float *>(rows);
+      for (int t0 = 0; t0 < n; t0 += 32) {
+        auto put = [&](int t, f32x4 y) {
+          if (g < 2)
+            *reinterpret_cast<f32x4 *>(yr + (t0 + 16 * t + r) * 8 + 4 * g) = y;
+        };
+        if (n - t0 > 16) {
+          const bf16x8 xs[2] = {input(t0), input(t0 + 16)};
+          infer_tiles<2>(sW, sBias, xs, put);
+        } else {
+          const bf16x8 xs[1] = {input(t0)};
+          infer_tiles<1>(sW, sBias, xs, put);
+        }
+      }
+      order();
+      if (net) {
+        float y[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) y[c] = yr[row * 8 + c];
+#pragma unroll
+        for (int c = 0; c < 8; c++)
+          y[c] = y[c] * jn * out_scale(c, rhos, cs) * area;
+        // back to the original frame
+        auto add = [&](auto d) {
+          constexpr int D = decltype(d)::value;
+          F[RHO] += y[0];
+#pragma unroll
+          for (int q = 0; q < 3; q++) {
+            F[MX + (D + q) % 3] += y[1 + q];
+            F[BX + (D + q) % 3] += y[4 + q];
+          }
+          F[EN] += y[7];
+        };
+        if (dir == 0) add(std::integral_constant<int, 0>());
+        else if (dir == 1) add(std::integral_constant<int, 1>());
+        else add(std::integral_constant<int, 2>());
+      }
+      order();
     }
+    if (valid)
+#pragma unroll
+      for (int v = 0; v < NSLOT; v++) a.face[(long)v * nTot + gf] = F[v];
   }
+  if (NET && lane == 0 && nNet) atomicAdd(&a.counters[0], nNet);
   if (err) atomicOr(a.err, err);
-  (void)nNet;
-}
-
-// the network on the compacted rows; fluxes back to the face array
-template <int NB>
-__global__ void __launch_bounds__(bats::mlp::kInferThreads, 8)
-k_sur_infer(const __bf16 *frag, const float *w, SurArgs a) {
-  using namespace bats::mlp;
-  using G = FaceGeom<NB>;
-  __shared__ __attribute__((aligned(16))) __bf16 sW[NFRAG];
-  __shared__ float sBias[NBIAS];
-  for (int t = threadIdx.x; t < NFRAG / 8; t += kInferThreads)
-    reinterpret_cast<bf16x8 *>(sW)[t] = reinterpret_cast<const bf16x8 *>(frag)[t];
-  load_biases(w, sBias);
-  __syncthreads();
-  const int rows = a.counters[0];
-  const int wave = threadIdx.x >> 6;
-  const long nTot = a.nFaceTot;
-  auto out = [&](int row, int c, float y) {
-    const int gf = a.rowFace[row];
-    const int dir = gf / (a.nBlock * G::NF);
-    const float4 sc = reinterpret_cast<const float4 *>(a.rowScale)[row];
-    const float area = sc.w;
-    const float v = y * sc.z * out_scale(c, sc.x, sc.y);
-    float &f = a.face[(long)rot_slot(dir, c) * nTot + gf];
-    f = f + v * area;
-  };
-  const int nTile = (rows + 15) / 16;
-  for (int tile = blockIdx.x * kInferWaves + wave; tile < nTile;
-       tile += gridDim.x * kInferWaves)
-    infer_tile(sW, sBias, a.rowX, rows, tile * 16, out);
 }
 
 // flux divergence and stage update (FP64), local time step; one workgroup
@@ -538,6 +563,14 @@ __global__ void __launch_bounds__(256) k_sur_update(SurArgs a) {
     if (threadIdx.x == 0)
       a.dtmaxB[b] = fmin2(fmin2(sRed[0], sRed[1]), fmin2(sRed[2], sRed[3]));
   }
+  // rows of this stage -> running totals
+  if (b == 0 && threadIdx.x == 0) {
+    *reinterpret_cast<unsigned long long *>(a.counters + 4) +=
+        (unsigned long long)a.counters[0];
+    *reinterpret_cast<unsigned long long *>(a.counters + 2) +=
+        (unsigned long long)a.nFaceTot;
+    a.counters[0] = 0;
+  }
   if (a.advanceTime && b == 0)
     for (int r = threadIdx.x; r < a.nRun; r += 256) {
       double *rr = a.scal + r * S_NSCAL;
@@ -582,16 +615,6 @@ k_sur_amr_correct(float *face, long nTot, int nBlock, const int *slabs,
 // counters: [0] rows of the current stage, [2..3] running total of faces
 // and [4..5] of network rows (64-bit), [1] unused
 constexpr int NCOUNTER = 6;
-__global__ void k_count_faces(int *counters, long nFace) {
-  // rows of this stage -> running totals (single thread)
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    atomicAdd(reinterpret_cast<unsigned long long *>(counters + 4),
-              (unsigned long long)counters[0]);
-    atomicAdd(reinterpret_cast<unsigned long long *>(counters + 2),
-              (unsigned long long)nFace);
-    counters[0] = 0;
-  }
-}
 
 }  // namespace
 
@@ -611,16 +634,19 @@ static void launch_harvest(int lim, int nB, hipStream_t st, const HarvestArgs &a
   }
 }
 
-template <int NB>
-static void launch_sur_faces(int lim, dim3 g, hipStream_t st, const SurArgs &a) {
-  const dim3 t(256);
-  switch (lim) {
-  case LIM_MINMOD: hipLaunchKernelGGL((k_sur_faces<NB, LIM_MINMOD>), g, t, 0, st, a); break;
-  case LIM_MC: hipLaunchKernelGGL((k_sur_faces<NB, LIM_MC>), g, t, 0, st, a); break;
-  case LIM_MC3: hipLaunchKernelGGL((k_sur_faces<NB, LIM_MC3>), g, t, 0, st, a); break;
-  case LIM_BETA: hipLaunchKernelGGL((k_sur_faces<NB, LIM_BETA>), g, t, 0, st, a); break;
-  case LIM_NO: hipLaunchKernelGGL((k_sur_faces<NB, LIM_NO>), g, t, 0, st, a); break;
-  default: hipLaunchKernelGGL((k_sur_faces<NB, LIM_FIRST>), g, t, 0, st, a); break;
+template <int NB, bool NET>
+static void launch_sur_faces(const SurArgs &a, hipStream_t st) {
+  constexpr int threads = NET ? kNetThreads : 256;
+  long nWg = (a.nFaceTot + threads - 1) / threads;
+  nWg = std::min(nWg, NET ? 512L : 16384L);
+  const dim3 g((unsigned)nWg), t(threads);
+  switch (a.lim) {
+  case LIM_MINMOD: hipLaunchKernelGGL((k_sur_faces<NB, LIM_MINMOD, NET>), g, t, 0, st, a); break;
+  case LIM_MC: hipLaunchKernelGGL((k_sur_faces<NB, LIM_MC, NET>), g, t, 0, st, a); break;
+  case LIM_MC3: hipLaunchKernelGGL((k_sur_faces<NB, LIM_MC3, NET>), g, t, 0, st, a); break;
+  case LIM_BETA: hipLaunchKernelGGL((k_sur_faces<NB, LIM_BETA, NET>), g, t, 0, st, a); break;
+  case LIM_NO: hipLaunchKernelGGL((k_sur_faces<NB, LIM_NO, NET>), g, t, 0, st, a); break;
+  default: hipLaunchKernelGGL((k_sur_faces<NB, LIM_FIRST, NET>), g, t, 0, st, a); break;
   }
 }
 
@@ -703,12 +729,9 @@ extern "C" int bats_set_surrogate(bats_handle *h, bats_mlp *m, int Mode,
   if (Mode != BATS_SUR_OFF && !s.face) {
     const long nF = (long)(h->NB + 1) * h->NB * h->NB;
     const long nTot = 3 * (long)h->cfg.nBlock * nF;
-    // rows and face indices are 32-bit (about 160k blocks of 16^3)
+    // face indices are 32-bit (about 160k blocks of 16^3)
     if (nTot > 0x7fffffffL) return BATS_ELIMIT;
     HIPCHK(hipMalloc(&s.face, sizeof(float) * NSLOT * nTot));
-    HIPCHK(hipMalloc(&s.rowX, sizeof(__bf16) * 16 * nTot));
-    HIPCHK(hipMalloc(&s.rowFace, sizeof(int) * nTot));
-    HIPCHK(hipMalloc(&s.rowScale, sizeof(float) * 4 * nTot));
     HIPCHK(hipMalloc(&s.counters, sizeof(int) * NCOUNTER));
     s.faceCap = nTot;
   }
@@ -774,24 +797,19 @@ int sur_stage(bats_handle *h, const StageArgs &sa) {
   a.advanceTime = sa.advanceTime;
   a.face = s.face;
   a.nFaceTot = s.faceCap;
-  a.rowX = s.rowX;
-  a.rowFace = s.rowFace;
-  a.rowScale = s.rowScale;
   a.counters = s.counters;
   const long nTot = s.faceCap;
-  long nWg = (nTot + 255) / 256;
-  if (nWg > 16384) nWg = 16384;
-  const int lim = sa.lim;
-  if (h->NB == 8) launch_sur_faces<8>(lim, dim3((unsigned)nWg), h->stream, a);
-  else launch_sur_faces<16>(lim, dim3((unsigned)nWg), h->stream, a);
+  a.frag = nullptr;
+  a.w = nullptr;
   if (s.mode == BATS_SUR_NETWORK) {
     const bats::mlp::Weights wts = bats::mlp::weights(s.model);
-    if (h->NB == 8)
-      hipLaunchKernelGGL(k_sur_infer<8>, dim3(bats::mlp::kInferGrid), dim3(bats::mlp::kInferThreads), 0, h->stream,
-                         wts.frag, wts.w, a);
-    else
-      hipLaunchKernelGGL(k_sur_infer<16>, dim3(bats::mlp::kInferGrid), dim3(bats::mlp::kInferThreads), 0, h->stream,
-                         wts.frag, wts.w, a);
+    a.frag = wts.frag;
+    a.w = wts.w;
+    if (h->NB == 8) launch_sur_faces<8, true>(a, h->stream);
+    else launch_sur_faces<16, true>(a, h->stream);
+  } else {
+    if (h->NB == 8) launch_sur_faces<8, false>(a, h->stream);
+    else launch_sur_faces<16, false>(a, h->stream);
   }
   if (h->nSlab > 0) {
     const long n = (long)h->nSlab * h->NB * h->NB;
@@ -807,8 +825,6 @@ int sur_stage(bats_handle *h, const StageArgs &sa) {
     hipLaunchKernelGGL(k_sur_update<8>, dim3(c.nBlock), dim3(256), 0, h->stream, a);
   else
     hipLaunchKernelGGL(k_sur_update<16>, dim3(c.nBlock), dim3(256), 0, h->stream, a);
-  hipLaunchKernelGGL(k_count_faces, dim3(1), dim3(64), 0, h->stream, s.counters,
-                     nTot);
   HIPCHK(hipGetLastError());
   return BATS_OK;
 }
