@@ -377,6 +377,14 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
   constexpr int NFL = BNLDS ? NFS + 2 : NFS;
   __shared__ T sP[BPW * NVAR * NR * NS];
   __shared__ T sF[BPW * 2 * NFL * NFX];
+  // areas of a block's x and y faces: FP64 without the 8-wave source reads
+  // them from LDS with the face's cells (4096 blocks of 16^3: 1480 -> 1456 us
+  // per launch); the 8-wave variants, at their register limit, and FP32 are
+  // 1-2 % faster with the cell sizes from global memory (384 and 392 us per
+  // launch on 512 blocks of 16^3 with body and B0, 226 and 228 us in FP32 on
+  // 1000)
+  constexpr bool AREALDS = sizeof(T) == 8 && !POWELL;
+  __shared__ T sArea[AREALDS ? BPW * 2 : 1];
   __shared__ double sRed[kThreads / 64];
 
   // steady state: a compile-time option of the plain variants, a run-time
@@ -507,6 +515,10 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
     const double dxb = a.cellsize[3 * bb], dyb = a.cellsize[3 * bb + 1],
                  dzb = a.cellsize[3 * bb + 2];
     const T AreaZ = T(dxb * dyb);
+    if (AREALDS && col == 0) {
+      sArea[2 * lb] = T(dyb * dzb);
+      sArea[2 * lb + 1] = T(dxb * dzb);
+    }
     // z sides of this block with DiLevel_EB /= 0 (wave-uniform)
     const bool zLo = RESB && a.nei[6 * bb + 4] < 0;
     const bool zHi = RESB && a.nei[6 * bb + 5] < 0;
@@ -628,6 +640,14 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
       }
     }
 
+    // the halo cell's place, looked up once for all planes (one plane further
+    // is NC cells on in a block, NB in a slab of ghost cells).  Looked up per
+    // plane, each wave ran up to four dependent neighbour loads and branches
+    // before its halo loads: FP64 HLLD on 4096 blocks of 16^3 1523 us per
+    // launch, 1495 us with the lookup here
+    const long hOff0 =
+        hAct ? cell_off<NB>(a.nei, hb, hii, hjj, 0, a.nCellTot) : 0;
+
     // plane k0-1 gives only the z face below plane k0: one copy of the z
     // face's code, so that a block split into parts rounds as a whole one
     for (int k = k0 - 1; k < k1; k++) {
@@ -658,7 +678,7 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
       // this thread's x/y halo cell of plane k
       if (hAct) {
         T q[NVAR];
-        load_state(U, vs, cell_off<NB>(a.nei, hb, hii, hjj, k, a.nCellTot), q);
+        load_state(U, vs, hOff0 + k * (hOff0 < a.nCellTot ? NC : NB), q);
         to_primitive(q);
 #pragma unroll
         for (int v = 0; v < NVAR; v++)
@@ -679,8 +699,6 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
         const int row = q / (NB + 1), fp = q % (NB + 1);
         T c0[NVAR], c1[NVAR], c2[NVAR], c3[NVAR];
         T F[NFLUX], vdt, unA;
-        const double dxf = a.cellsize[3 * bf], dyf = a.cellsize[3 * bf + 1],
-                     dzf = a.cellsize[3 * bf + 2];
         // y faces are evaluated as x faces of the cyclically rotated frame
         // (x, y, z) -> (y, z, x): the same normal / tangent1 / tangent2
         // order as the y-normal flux, so a wave whose faces mix x and y runs
@@ -698,7 +716,13 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
           c2[v] = sP[o + 2 * st];
           c3[v] = sP[o + 3 * st];
         }
-        const T area = T(dir == 0 ? dyf * dzf : dxf * dzf);
+        T area;
+        if (AREALDS) {
+          area = sArea[2 * lbf + dir];
+        } else {
+          const double *cs = a.cellsize + 3 * bf;
+          area = T(dir == 0 ? cs[1] * cs[2] : cs[0] * cs[2]);
+        }
         T bL = beta, bR = beta;
         if (RESB) {
           const bool lo = a.nei[6 * bf + 2 * dir] < 0;
@@ -991,9 +1015,12 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
 #pragma unroll
             for (int v = 0; v < NVAR; v++) Uod[v] = double(Uo[v]);
             if (uc.dtZero || !uc.halfStep) {
-              load_state(U, vs, off, Uc);
+              // the window's own entry, whose primitive form differs from it
+              // in the momentum alone (five loads of eight left out: 1495 ->
+              // 1480 us at the size above)
 #pragma unroll
-              for (int v = 0; v < NVAR; v++) Ucd[v] = double(Uc[v]);
+              for (int v = 0; v < NVAR; v++)
+                Ucd[v] = double(v >= MX && v <= MZ ? U[v * vs + off] : Q1[v]);
               update_cell(a.ph, ucc, dF, Ucd, Uod, Un);
             } else {
               update_cell(a.ph, ucc, dF, Uod, Uod, Un);
