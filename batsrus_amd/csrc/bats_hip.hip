@@ -1917,6 +1917,17 @@ static void tvd_args(const bats_handle *h, AmrArgs &m) {
   m.tvdBeta = std::min(c.BetaLimiterResChange, c.LimiterBeta);
 }
 
+// one variable per thread; with the TVD treatment, whose restriction mixes
+// the variables, all of a cell's
+template <int NB, typename T>
+static void launch_ghosts(const AmrArgs &m, long n, hipStream_t st) {
+  const unsigned g = (unsigned)((n + 255) / 256);
+  if (m.tvd)
+    hipLaunchKernelGGL((k_amr_ghosts<NB, T, NVAR>), dim3(g), dim3(256), 0, st, m);
+  else
+    hipLaunchKernelGGL((k_amr_ghosts<NB, T, 1>), dim3(g, NVAR), dim3(256), 0, st, m);
+}
+
 int amr_fill_ghosts(bats_handle *h, const void *U) {
   AmrArgs m{};
   tvd_args(h, m);
@@ -1934,11 +1945,9 @@ int amr_fill_ghosts(bats_handle *h, const void *U) {
   m.corr = h->corr; m.err = h->err; m.bcState = h->dBcState;
   m.pOutflow = h->cfg.pOutflow;
   const long n = 2L * h->NB * h->NB * h->nSlab;
-  const dim3 g((unsigned)((n + 255) / 256)), t(256);
-  if (h->elemSize == 8)
-    hipLaunchKernelGGL(k_amr_ghosts<double>, g, t, 0, h->stream, m, h->NB);
-  else
-    hipLaunchKernelGGL(k_amr_ghosts<float>, g, t, 0, h->stream, m, h->NB);
+  const bool f64 = h->elemSize == 8;
+  if (h->NB == 8) f64 ? launch_ghosts<8, double>(m, n, h->stream) : launch_ghosts<8, float>(m, n, h->stream);
+  else f64 ? launch_ghosts<16, double>(m, n, h->stream) : launch_ghosts<16, float>(m, n, h->stream);
   HIPCHK(hipGetLastError());
   return BATS_OK;
 }

@@ -1158,19 +1158,37 @@ __device__ __forceinline__ T minmod2(T a, T b) {
 // src/ModCellBoundary.f90:308-331,624-666); kind-4 slabs (outflow sides
 // with a fixed pressure) copy the boundary cell and set the pressure
 // (src/ModCellBoundary.f90:273-277).  One thread per ghost cell.
-template <typename T>
-__global__ void __launch_bounds__(256) k_amr_ghosts(AmrArgs a, int NB) {
-  const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  const long per = 2L * NB * NB;
-  if (t >= per * a.nSlab) return;
-  const int slab = (int)(t / per), r = (int)(t % per);
+//
+// Bound by the latency of its loads, one line each on x sides, with few cells
+// in all (a block's side has 2 NB^2): the variables v0 .. v0+VG-1 of a cell
+// are a thread's work, so that its loads are all under way together and the
+// chip is full.  VG = NVAR with the TVD treatment, whose restriction mixes the
+// variables.  A wave's cells lie in one slab: its record and the branches on
+// its kind are the wave's.  800 slabs of 8^3 blocks: 25.1 us with one thread
+// for all variables, 15.6 us with VG = 2, 11.7 us with VG = 1 (FP32 21.4 us and
+// 10.0 us).
+template <int NB, typename T, int VG>
+__global__ void __launch_bounds__(256) k_amr_ghosts(AmrArgs a) {
+  constexpr int per = 2 * NB * NB;
+  static_assert(per % 64 == 0, "one slab per wave");
+  const int slab = __builtin_amdgcn_readfirstlane(
+      (int)((blockIdx.x * 256L + threadIdx.x) / per));
+  if (slab >= a.nSlab) return;
+  const int r = (blockIdx.x * 256 + threadIdx.x) % per;
+  const int v0 = VG == NVAR ? 0 : blockIdx.y * VG;
   const int L = r / (NB * NB), q = (r / NB) % NB, p = r % NB;
   const int *sl = a.slabs + 8 * slab;
-  const int side = sl[1], kind = sl[2], d = side / 2, hi = side % 2, H = NB / 2;
-  const T *U = static_cast<const T *>(a.U);
-  T val[NVAR];
+  const int side = sl[1], kind = sl[2], d = side / 2, hi = side % 2;
+  constexpr int H = NB / 2;
+  const long vs = a.vs;
+  const T *U = static_cast<const T *>(a.U) + v0 * vs;
+  T val[VG];
   auto cell = [&](int blk, int x, int y, int z) {
     return (((long)blk * NB + z) * NB + y) * NB + x;
+  };
+  auto load = [&](long o) {
+#pragma unroll
+    for (int v = 0; v < VG; v++) val[v] = U[v * vs + o];
   };
   if (kind == 2 || kind == 5) {
     if (kind == 5 && a.nVary > 0) {
@@ -1197,34 +1215,40 @@ __global__ void __launch_bounds__(256) k_amr_ghosts(AmrArgs a, int NB) {
                  Dx * (a.varyS[(lo + 1) * NVAR + v] - a.varyS[lo * NVAR + v]);
       }
       for (int v = MX; v <= MZ; v++) w[v] = w[v] * w[RHO];
-      for (int v = 0; v < NVAR; v++) val[v] = T(w[v]);
+#pragma unroll
+      for (int c = 0; c < NVAR; c++)
+        if (c >= v0 && c < v0 + VG) val[c % VG] = T(w[c]);
     } else {
-      for (int v = 0; v < NVAR; v++) val[v] = T(a.bcState[side * NVAR + v]);
+#pragma unroll
+      for (int v = 0; v < VG; v++) val[v] = T(a.bcState[side * NVAR + v0 + v]);
     }
     if (a.b0SideSlot) {
       const int slot = a.b0SideSlot[6 * sl[0] + side];
       if (slot >= 0) {
         const double *b0 = a.b0Side + (((long)slot * 2 + L) * NB * NB +
                                        (long)q * NB + p) * 3;
-        for (int c = 0; c < 3; c++)
-          val[BX + c] = T(double(val[BX + c]) - b0[c]);
+#pragma unroll
+        for (int v = 0; v < VG; v++) {
+          const int c = v0 + v - BX;
+          if (c >= 0 && c < 3) val[v] = T(double(val[v]) - b0[c]);
+        }
       }
     }
   } else if (kind == 4) {
     int x, y, z;
     side_xyz(d, hi ? NB - 1 : 0, p, q, x, y, z);
-    const long o = cell(sl[0], x, y, z);
-    for (int v = 0; v < NVAR; v++) val[v] = U[v * a.vs + o];
-    val[PP] = T(a.pOutflow);
+    load(cell(sl[0], x, y, z));
+#pragma unroll
+    for (int v = 0; v < VG; v++)
+      if (v0 + v == PP) val[v] = T(a.pOutflow);
   } else if (kind == 3) {
     int x, y, z;
     side_xyz(d, hi ? NB - 1 - L : L, p, q, x, y, z);
-    const long o = cell(sl[0], x, y, z);
-    for (int v = 0; v < NVAR; v++) {
-      const T u = U[v * a.vs + o];
-      val[v] = (v == MX + d || v == BX + d) ? -u : u;
-    }
-  } else if (kind == 1 && a.tvd) {
+    load(cell(sl[0], x, y, z));
+#pragma unroll
+    for (int v = 0; v < VG; v++)
+      if (v0 + v == MX + d || v0 + v == BX + d) val[v] = -val[v];
+  } else if (VG == NVAR && kind == 1) {
     // face restriction: the 2x2 fine cells of the fine layer nearest to
     // the ghost layer (DoRestrictFace, src/ModMessagePass.f90:105); layer 0
     // moves to the coarse cell distance from the block's own cell in
@@ -1233,49 +1257,64 @@ __global__ void __launch_bounds__(256) k_amr_ghosts(AmrArgs a, int NB) {
     // coarse face it serves takes the fine fluxes.
     const int F = sl[3 + (p / H) + 2 * (q / H)];
     const int nf = hi ? 2 * L : NB - 1 - 2 * L;
-    for (int v = 0; v < NVAR; v++) val[v] = T(0);
+#pragma unroll
+    for (int v = 0; v < VG; v++) val[v] = T(0);
+#pragma unroll
     for (int bq = 0; bq < 2; bq++)
+#pragma unroll
       for (int cp = 0; cp < 2; cp++) {
         int x, y, z;
         side_xyz(d, nf, 2 * (p % H) + cp, 2 * (q % H) + bq, x, y, z);
         const long o = cell(F, x, y, z);
-        for (int v = 0; v < NVAR; v++) val[v] += U[v * a.vs + o];
+#pragma unroll
+        for (int v = 0; v < VG; v++) val[v] += U[v * vs + o];
       }
-    for (int v = 0; v < NVAR; v++) val[v] = T(0.25) * val[v];
-    if (L == 0 && a.twoLayers) {
-      int x, y, z;
-      side_xyz(d, hi ? NB - 1 : 0, p, q, x, y, z);
-      T c[NVAR];
-      load_state(U, a.vs, cell(sl[0], x, y, z), c);
-      to_primitive(c);
-      to_primitive(val);
-      const T cThird = T(1.0 / 3.0);
-      for (int v = 0; v < NVAR; v++) val[v] = val[v] + cThird * (val[v] - c[v]);
-      val[RHO] = fmax2(val[RHO], T(1e-30));
-      val[PP] = fmax2(val[PP], T(1e-30));
-      for (int v = MX; v <= MZ; v++) val[v] = val[v] * val[RHO];
-    }
-  } else if (kind == 0 && a.tvd) {
+#pragma unroll
+    for (int v = 0; v < VG; v++) val[v] = T(0.25) * val[v];
+    if constexpr (VG == NVAR)
+      if (L == 0 && a.twoLayers) {
+        int x, y, z;
+        side_xyz(d, hi ? NB - 1 : 0, p, q, x, y, z);
+        T c[NVAR];
+        load_state(U, vs, cell(sl[0], x, y, z), c);
+        to_primitive(c);
+        to_primitive(val);
+        const T cThird = T(1.0 / 3.0);
+#pragma unroll
+        for (int v = 0; v < NVAR; v++)
+          val[v] = val[v] + cThird * (val[v] - c[v]);
+        val[RHO] = fmax2(val[RHO], T(1e-30));
+        val[PP] = fmax2(val[PP], T(1e-30));
+#pragma unroll
+        for (int v = MX; v <= MZ; v++) val[v] = val[v] * val[RHO];
+      }
+  } else if (VG == NVAR && kind == 0) {
     // first-order prolongation: the coarse cell itself; with the
     // second-order scheme the two ghost layers take the two coarse layers
     // behind the face (DoTwoCoarseLayers, src/ModMessagePass.f90:108-109)
     const int Lc = a.twoLayers ? L : 0;
     int x, y, z;
     side_xyz(d, hi ? Lc : NB - 1 - Lc, sl[4] + p / 2, sl[5] + q / 2, x, y, z);
-    load_state(U, a.vs, cell(sl[3], x, y, z), val);
+    load(cell(sl[3], x, y, z));
   } else if (kind == 1) {
     const int F = sl[3 + (p / H) + 2 * (q / H)];
-    for (int v = 0; v < NVAR; v++) val[v] = T(0);
+#pragma unroll
+    for (int v = 0; v < VG; v++) val[v] = T(0);
+#pragma unroll
     for (int ai = 0; ai < 2; ai++)
+#pragma unroll
       for (int bq = 0; bq < 2; bq++)
+#pragma unroll
         for (int cp = 0; cp < 2; cp++) {
           const int nf = hi ? 2 * L + ai : NB - 1 - 2 * L - ai;
           int x, y, z;
           side_xyz(d, nf, 2 * (p % H) + cp, 2 * (q % H) + bq, x, y, z);
           const long o = cell(F, x, y, z);
-          for (int v = 0; v < NVAR; v++) val[v] += U[v * a.vs + o];
+#pragma unroll
+          for (int v = 0; v < VG; v++) val[v] += U[v * vs + o];
         }
-    for (int v = 0; v < NVAR; v++) val[v] = T(0.125) * val[v];
+#pragma unroll
+    for (int v = 0; v < VG; v++) val[v] = T(0.125) * val[v];
   } else {
     const int C = sl[3];
     int cc[3];
@@ -1289,51 +1328,73 @@ __global__ void __launch_bounds__(256) k_amr_ghosts(AmrArgs a, int NB) {
     else if (d == 1) { delta[0] = dp; delta[1] = dn; delta[2] = dq; }
     else { delta[0] = dp; delta[1] = dq; delta[2] = dn; }
     const long o0 = cell(C, cc[0], cc[1], cc[2]);
-    for (int v = 0; v < NVAR; v++) val[v] = U[v * a.vs + o0];
+    load(o0);
+    T u0[VG];
+#pragma unroll
+    for (int v = 0; v < VG; v++) u0[v] = val[v];
+#pragma unroll
     for (int dd = 0; dd < 3; dd++) {
-      int lo[3] = {cc[0], cc[1], cc[2]}, up[3] = {cc[0], cc[1], cc[2]};
-      lo[dd] -= 1;
-      up[dd] += 1;
+      constexpr int step[3] = {1, NB, NB * NB};
       const bool hasLo = cc[dd] > 0, hasUp = cc[dd] < NB - 1;
-      const long ol = hasLo ? cell(C, lo[0], lo[1], lo[2]) : o0;
-      const long ou = hasUp ? cell(C, up[0], up[1], up[2]) : o0;
-      for (int v = 0; v < NVAR; v++) {
-        const T u0 = U[v * a.vs + o0];
+      const long ol = hasLo ? o0 - step[dd] : o0;
+      const long ou = hasUp ? o0 + step[dd] : o0;
+#pragma unroll
+      for (int v = 0; v < VG; v++) {
+        const T lo = u0[v] - U[v * vs + ol], up = U[v * vs + ou] - u0[v];
         T g = T(0);
-        if (hasLo && hasUp) g = minmod2(u0 - U[v * a.vs + ol], U[v * a.vs + ou] - u0);
-        else if (hasLo) g = u0 - U[v * a.vs + ol];
-        else if (hasUp) g = U[v * a.vs + ou] - u0;
+        if (hasLo && hasUp) g = minmod2(lo, up);
+        else if (hasLo) g = lo;
+        else if (hasUp) g = up;
         val[v] = val[v] + g * delta[dd];
       }
     }
   }
   T *W = const_cast<T *>(U);
   const long o = a.nCellTot + ((long)slab * 2 + L) * NB * NB + (long)q * NB + p;
-  for (int v = 0; v < NVAR; v++) W[v * a.vs + o] = val[v];
+#pragma unroll
+  for (int v = 0; v < VG; v++) W[v * vs + o] = val[v];
 }
 
 // save_cons_flux (src/ModConserveFlux.f90:79-187): the face fluxes of the
 // fine blocks at their coarser sides, into the coarse slab's store at
-// (coarse face, sub-face) -- one thread per fine face
+// (coarse face, sub-face) -- one thread per fine face.  Few faces, a long
+// chain each: one wave per workgroup puts them on all CUs, and a wave's faces
+// lie in one slab, whose record and cell places are the wave's.  640 slabs of
+// 8^3 blocks: 12.3 us with four waves per workgroup and a neighbour lookup
+// per cell, 10.9 us so.
+constexpr int kFineThreads = 64;
+
 template <int NB, int FLUX, int LIM, typename T>
-__global__ void __launch_bounds__(256) k_amr_fineflux(AmrArgs a) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(kFineThreads) k_amr_fineflux(AmrArgs a) {
+  const int t = blockIdx.x * kFineThreads + threadIdx.x;
   if (t >= a.nFine * NB * NB) return;
-  const int slab = a.fineSlabs[t / (NB * NB)];
+  static_assert(NB * NB % kFineThreads == 0, "one slab per wave");
+  const int slab =
+      __builtin_amdgcn_readfirstlane(a.fineSlabs[t / (NB * NB)]);
   const int q = (t / NB) % NB, p = t % NB;
   const int *sl = a.slabs + 8 * slab;
   const int b = sl[0], side = sl[1], d = side / 2, hi = side % 2;
   const T *U = static_cast<const T *>(a.U);
   const PhysT<T> ph = phys_as<T>(a.ph);
   T c[4][NVAR];
+#pragma unroll
   for (int s4 = 0; s4 < 4; s4++) {
-    // face between normal cells f-1 and f; f = 0 (low side) or NB (high)
+    // face between normal cells f-1 and f; f = 0 (low side) or NB (high):
+    // two cells of the block, two of the slab's layers
     const int nrm = (hi ? NB : 0) + s4 - 2;
-    int x, y, z;
-    side_xyz(d, nrm, p, q, x, y, z);
-    load_state(U, a.vs, cell_off<NB>(a.nei, b, x, y, z, a.nCellTot), c[s4]);
-    to_primitive(c[s4]);
+    long o;
+    if (nrm < 0 || nrm >= NB) {
+      o = a.nCellTot +
+          (((long)slab * 2 + (hi ? nrm - NB : -1 - nrm)) * NB + q) * NB + p;
+    } else {
+      int x, y, z;
+      side_xyz(d, nrm, p, q, x, y, z);
+      o = (((long)b * NB + z) * NB + y) * NB + x;
+    }
+    load_state(U, a.vs, o, c[s4]);
   }
+#pragma unroll
+  for (int s4 = 0; s4 < 4; s4++) to_primitive(c[s4]);
   const double *cz = a.cellsize + 3 * b;
   const T area = T(d == 0 ? cz[1] * cz[2] : d == 1 ? cz[0] * cz[2] : cz[0] * cz[1]);
   T L[NVAR], R[NVAR], F[NFLUX], vdt, unA;
@@ -1461,7 +1522,7 @@ __global__ void __launch_bounds__(256) k_amr_fineflux(AmrArgs a) {
 
 template <int NB, int FLUX, typename T>
 inline hipError_t launch_amr_fineflux(const AmrArgs &a, hipStream_t stream) {
-  const dim3 grid((a.nFine * NB * NB + 255) / 256), block(256);
+  const dim3 grid(a.nFine * NB * NB / kFineThreads), block(kFineThreads);
   switch (a.lim) {
   case LIM_MINMOD: hipLaunchKernelGGL((k_amr_fineflux<NB, FLUX, LIM_MINMOD, T>), grid, block, 0, stream, a); break;
   case LIM_MC: hipLaunchKernelGGL((k_amr_fineflux<NB, FLUX, LIM_MC, T>), grid, block, 0, stream, a); break;
