@@ -326,13 +326,44 @@ struct SurArgs {
 // KiB with the rows on their way, two workgroups per CU, four waves per SIMD)
 constexpr int kNetThreads = 512;
 
+// The four cells along the normal of face (fi, fj, fk).  At most one side of
+// the block is near, so that one neighbour is looked up and the loads of all
+// cells are under way together (815 -> 805 us per stage at the size below; a
+// lookup per cell waited for the loads of the cells before it).
+template <int NB>
+__device__ __forceinline__ void face_cells(const int *__restrict__ nei, int b,
+                                           int dir, int fi, int fj, int fk,
+                                           long nCellTot, long *off) {
+  const int f = dir == 0 ? fi : dir == 1 ? fj : fk;
+  const int p = dir == 0 ? fj : fi, q = dir == 2 ? fj : fk;
+  const int st = dir == 0 ? 1 : dir == 1 ? NB : NB * NB;
+  const bool hi = f >= NB / 2;
+  const long o = (((long)b * NB + fk) * NB + fj) * NB + fi;
+  const int n = f < 2 || f > NB - 2 ? nei[6 * b + 2 * dir + hi] : 0;
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    const int c = f + s - 2;  // the cell's place along the normal
+    off[s] = o + (s - 2) * st;
+    if (c < 0 || c >= NB) {
+      if (n >= 0)
+        off[s] += (long)(n - b) * (NB * NB * NB) + (hi ? -NB : NB) * st;
+      else if (n == -1)
+        off[s] = o + ((hi ? NB - 1 : 0) - f) * st;
+      else
+        off[s] = nCellTot +
+                 (((long)(-2 - n) * 2 + (hi ? c - NB : -1 - c)) * NB + q) * NB +
+                 p;
+    }
+  }
+}
+
 // One face per lane.  NET: a wave packs the inputs of its faces that passed
 // the gate into rows in LDS, takes them through the network 32 at a time and
 // adds each correction to the flux its lane still holds, so a face's flux is
 // written once and no input, scale or index of it ever.  The two together
 // are bound by the vector unit (SiLU's two transcendentals per activation);
 // apart, the rows cost 204 bytes of memory traffic per face: 722 + 328 us per
-// stage at 6.7 million faces, 818 us now.
+// stage at 6.7 million faces, 815 us as one kernel.
 template <int NB, int LIM, bool NET>
 __global__ void __launch_bounds__(NET ? kNetThreads : 256, NET ? 4 : 1)
 k_sur_faces(SurArgs a) {
@@ -373,12 +404,12 @@ k_sur_faces(SurArgs a) {
       int fi, fj, fk;
       G::decode(dir, r, fi, fj, fk);
       float q[4][NVAR];
-      for (int s = 0; s < 4; s++) {
-        int ii = fi, jj = fj, kk = fk;
-        if (dir == 0) ii += s - 2; else if (dir == 1) jj += s - 2; else kk += s - 2;
-        load_state(a.Uin, a.vs, cell_off<NB>(a.nei, b, ii, jj, kk, a.nCellTot), q[s]);
-        to_primitive(q[s]);
-      }
+      long off[4];
+      face_cells<NB>(a.nei, b, dir, fi, fj, fk, a.nCellTot, off);
+#pragma unroll
+      for (int s = 0; s < 4; s++) load_state(a.Uin, a.vs, off[s], q[s]);
+#pragma unroll
+      for (int s = 0; s < 4; s++) to_primitive(q[s]);
       float L[NVAR], R[NVAR];
       face_states<LIM>(beta, beta, q[0], q[1], q[2], q[3], L, R);
       const double *cz = a.cellsize + 3 * b;
