@@ -6,15 +6,14 @@ state, and keeps the fastest:
   * cells per thread: each thread marches NB, NB/2 or NB/4 planes of its
     column (the block's planes split over 1, 2 or 4 workgroups, which
     fills more of the chip on small grids at the price of one more z-face
-    row per part; the face at each part boundary is evaluated by the
-    window's prologue, which rounds within an ulp of the in-loop face);
+    row per part);
   * work order: linear, or XCD-contiguous (each of the 8 XCDs takes a
     contiguous range of the Morton-ordered work list, so neighbouring
     blocks share its L2);
   * the persistent work-list grid size (0 = one workgroup per work item,
     else a multiple of the 256 compute units);
   * the per-step hipGraph.
-All shapes but the cells per thread leave the results bit-identical.
+All shapes give the same bits.
 Results are stored in a JSON file keyed by the device, the block size, the
 scheme and the grid shape, so later runs of the same workload apply the
 stored choice without timing again.

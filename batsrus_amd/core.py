@@ -529,8 +529,9 @@ class Session:
 
     def set_stage_shape(self, CellsPerThread=None, UseXcdOrder=False):
         """Cells per thread of the stage kernel (NB, NB/2 or NB/4; None:
-        NB) and the XCD-contiguous work order (the same bits; a split
-        rounds its part-boundary faces within an ulp)."""
+        NB) and the XCD-contiguous work order (the same bits for every
+        shape).  A session without a call leaves the cells per thread to
+        the library, which chooses from the number of blocks."""
         cpt = self.grid.nI if CellsPerThread is None else int(CellsPerThread)
         self._check(self.lib.bats_set_stage_shape(self.h, cpt,
                                                   int(bool(UseXcdOrder))),

@@ -571,12 +571,6 @@ k_global_dt(const double *dtmaxB, const int *runFirst, double *scalAll,
   }
 }
 
-// fill n doubles with v
-__global__ void __launch_bounds__(256) k_fill(double *p, long n, double v) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) p[t] = v;
-}
-
 template <typename T>
 __global__ void k_check_nan(const T *U, long n, int *err) {
   int bad = 0;
@@ -705,9 +699,12 @@ extern "C" int bats_init(const bats_config *cfg, bats_handle **out) {
     if (e == hipSuccess) e = hipMalloc(&h->U[u], sz);
   if (e == hipSuccess) e = hipMalloc(&h->nei, sizeof(int) * 6 * c.nBlock);
   if (e == hipSuccess) e = hipMalloc(&h->cellsize, sizeof(double) * 3 * c.nBlock);
-  if (e == hipSuccess) e = hipMalloc(&h->dtmaxB, sizeof(double) * c.nBlock);
-  if (e == hipSuccess) e = hipMalloc(&h->dtAcc, sizeof(*h->dtAcc) * c.nBlock);
-  if (e == hipSuccess) e = hipMalloc(&h->dtCnt, sizeof(*h->dtCnt) * c.nBlock);
+  // the blocks' time steps and what the parts of a split block meet in:
+  // dtmaxB, dtAcc and dtCnt in one allocation, set by one copy
+  const size_t nDt = c.nBlock, szDt = (2 * sizeof(double) + sizeof(unsigned)) * nDt;
+  if (e == hipSuccess) e = hipMalloc(&h->dtmaxB, szDt);
+  h->dtAcc = reinterpret_cast<unsigned long long *>(h->dtmaxB + nDt);
+  h->dtCnt = reinterpret_cast<unsigned *>(h->dtAcc + nDt);
   if (e == hipSuccess) e = hipMalloc(&h->scal, sizeof(double) * S_NSCAL);
   if (e == hipSuccess) e = hipMalloc(&h->runFirst, sizeof(int) * 2);
   if (e == hipSuccess) e = hipMalloc(&h->runOfBlock, sizeof(int) * c.nBlock);
@@ -741,12 +738,9 @@ extern "C" int bats_init(const bats_config *cfg, bats_handle **out) {
                    hipMemcpyHostToDevice));
   HIPCHK(hipMemset(h->runOfBlock, 0, sizeof(int) * c.nBlock));
   HIPCHK(hipMemset(h->err, 0, sizeof(int)));
-  HIPCHK(hipMemset(h->dtmaxB, 0, sizeof(double) * c.nBlock));
-  HIPCHK(hipMemset(h->dtCnt, 0, sizeof(*h->dtCnt) * c.nBlock));
-  hipLaunchKernelGGL(k_fill, dim3((c.nBlock + 255) / 256), dim3(256), 0,
-                     h->stream, reinterpret_cast<double *>(h->dtAcc),
-                     (long)c.nBlock, 1.7976931348623157e308);
-  HIPCHK(hipGetLastError());
+  std::vector<double> dt0((szDt + 7) / 8, 0.0);
+  std::fill(dt0.begin() + nDt, dt0.begin() + 2 * nDt, 1.7976931348623157e308);
+  HIPCHK(hipMemcpy(h->dtmaxB, dt0.data(), szDt, hipMemcpyHostToDevice));
   h->splitShift = -1;
   // outer boundaries float until bats_set_cell_boundary
   for (int side = 0; side < 6; side++) h->bcType[side] = BATS_BC_FLOAT;
@@ -772,7 +766,7 @@ extern "C" int bats_finalize(bats_handle *h) {
   if (!h) return BATS_EINVAL;
   (void)hipStreamSynchronize(h->stream);
   void *ptrs[] = {h->U[0], h->U[1], h->U[2], h->Usnap, h->nei, h->cellsize, h->dtmaxB,
-                  h->dtmaxCB, h->dtAcc, h->dtCnt, h->scal, h->runFirst, h->runOfBlock, h->err,
+                  h->dtmaxCB, h->scal, h->runFirst, h->runOfBlock, h->err,
                   h->partial, h->LX, h->RX,
                   h->LY, h->RY, h->LZ, h->RZ, h->FX, h->FY, h->FZ, h->Src,
                   h->sur.face, h->sur.counters, h->slabs, h->slabKind, h->fineSlabs,
@@ -1893,8 +1887,7 @@ extern "C" int bats_set_persistent_grid(bats_handle *h, int nWorkgroup) {
 }
 
 // cells per thread of the stage kernel (NB, NB/2 or NB/4 planes of each
-// column per work item) and the XCD-contiguous work order (the same bits;
-// a split rounds the part-boundary faces within an ulp)
+// column per work item) and the XCD-contiguous work order (the same bits)
 extern "C" int bats_set_stage_shape(bats_handle *h, int CellsPerThread,
                                     int UseXcdOrder) {
   if (!h) return BATS_EINVAL;
