@@ -431,6 +431,10 @@ __global__ void k_pack_frag(const float *w, __bf16 *frag, __bf16 *bfrag) {
 
 namespace {
 
+// Bound by the vector unit (SiLU) on many rows and on few by the copy of the
+// weights into LDS, after which each wave has one pair of tiles: 65,536 rows
+// in 15.8 us, as with 16 waves of one tile each at 64 VGPRs (15.7 us), which
+// spill with the pair that the surrogate's faces need.
 __global__ void __launch_bounds__(kInferThreads, 4)
 k_infer(const __bf16 *frag, const float *w, const float *X, float *Y,
         int rows) {
@@ -441,7 +445,7 @@ k_infer(const __bf16 *frag, const float *w, const float *X, float *Y,
   load_biases(w, sBias);
   __syncthreads();
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const int nPair = (rows + 31) / 32;
+  const int nPair = (rows - 1) / 32 + 1;
   for (int pair = blockIdx.x * kInferWaves + (threadIdx.x >> 6); pair < nPair;
        pair += gridDim.x * kInferWaves) {
     bf16x8 x[2];
@@ -762,7 +766,7 @@ int bats::mlp::forward_device(bats_mlp *m, const float *dX, float *dY,
   int st = repack(m);
   if (st) return st;
   MCHK(hipStreamSynchronize(m->stream));
-  const int nPair = (rows + 31) / 32;
+  const int nPair = (rows - 1) / 32 + 1;
   int grid = (nPair + kInferWaves - 1) / kInferWaves;
   if (grid > kInferGrid) grid = kInferGrid;
   hipLaunchKernelGGL(k_infer, dim3(grid), dim3(kInferThreads), 0, stream, m->frag, m->w,

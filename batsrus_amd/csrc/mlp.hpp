@@ -116,7 +116,7 @@ __device__ __forceinline__ float dsilu(float z) {
 
 // =====================================================================
 // batched inference: Y[rows x 8] = MLP(X[rows x 16]) with fragment-ordered
-// BF16 weights (flat FP32 biases); a workgroup walks 64-row groups
+// BF16 weights (flat FP32 biases); a wave takes 32 rows at a time
 // =====================================================================
 // inference workgroups: 8 waves share one LDS copy of the weights (59 KiB);
 // two workgroups per CU, 4 waves per SIMD (at most 128 VGPRs)
