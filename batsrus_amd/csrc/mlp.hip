@@ -465,17 +465,48 @@ k_infer(const __bf16 *frag, const float *w, const float *X, float *Y,
   }
 }
 
-__global__ void k_gather_rows_f32(const float *dataX, const float *dataT,
-                                  const float *dataB, const float *dataJ,
-                                  const int *idx, int B, float *X, float *T,
-                                  float *Bo, float *Jo) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= B) return;
-  const long s = idx[t];
-  for (int j = 0; j < 16; j++) X[(long)t * 16 + j] = dataX[s * 16 + j];
-  for (int j = 0; j < 8; j++) T[(long)t * 8 + j] = dataT[s * 8 + j];
-  for (int j = 0; j < 8; j++) Bo[(long)t * 8 + j] = dataB[s * 8 + j];
-  Jo[t] = dataJ[s];
+// the inputs of listed samples, one value per thread
+__global__ void __launch_bounds__(256)
+k_gather_inputs(const float *X, const int *idx, int rows, float *Xo) {
+  const long t = blockIdx.x * 256L + threadIdx.x;
+  if (t < rows * 16L) Xo[t] = X[idx[t / 16] * 16L + t % 16];
+}
+
+// The held-out errors: for output j = thread % 8 the sums over the listed
+// samples of (w (Y - T))^2, (w T + B)^2 and (w T)^2 in FP64, w the sample's
+// jump norm (predicted flux B + w Y against the full flux B + w T); per
+// workgroup part[3][8], summed on the host in their order.  Bound by its
+// reads (100 bytes per sample).  With the gathered samples copied to the host
+// and summed there, a call that trains nothing on 700,001 samples took
+// 2.9 ms, 1.9 ms so (four epochs of them 10.7 -> 9.8 ms).
+constexpr int kErrGrid = 256;
+__global__ void __launch_bounds__(256)
+k_hold_err(const float *Y, const float *T, const float *B, const float *J,
+           const int *idx, int rows, double *part) {
+  __shared__ double sSum[4][3][8];
+  const int j = threadIdx.x & 7;
+  double sum[3] = {0.0, 0.0, 0.0};
+  for (long r = blockIdx.x * 32L + threadIdx.x / 8; r < rows;
+       r += gridDim.x * 32L) {
+    const long s = idx[r];
+    const double w = J[s], t = T[s * 8 + j];
+    const double d = w * ((double)Y[r * 8 + j] - t);
+    const double wt = w * t, f = wt + (double)B[s * 8 + j];
+    sum[0] += d * d;
+    sum[1] += f * f;
+    sum[2] += wt * wt;
+  }
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+#pragma unroll
+    for (int o = 8; o < 64; o *= 2) sum[q] += __shfl_xor(sum[q], o);
+    if ((threadIdx.x & 63) < 8) sSum[threadIdx.x / 64][q][j] = sum[q];
+  }
+  __syncthreads();
+  if (threadIdx.x < 24) {
+    const double *p = &sSum[0][0][0] + threadIdx.x;
+    part[blockIdx.x * 24 + threadIdx.x] = ((p[0] + p[24]) + p[48]) + p[72];
+  }
 }
 
 }  // namespace
@@ -1052,57 +1083,42 @@ extern "C" int bats_mlp_train(bats_mlp *m, int nEpoch, int Batch, double Lr0,
   if (TrainLoss) *TrainLoss = lastLoss;
   // held-out relative error: ||Y - T|| / ||T|| overall and per output
   if (HeldOutRelErr_V && nHold > 0) {
-    float *hx = nullptr, *ht = nullptr, *hy = nullptr, *hb = nullptr,
-          *hj = nullptr;
-    MCHK(hipMalloc(&hx, sizeof(float) * (size_t)nHold * 16));
-    MCHK(hipMalloc(&ht, sizeof(float) * (size_t)nHold * 8));
-    MCHK(hipMalloc(&hy, sizeof(float) * (size_t)nHold * 8));
-    MCHK(hipMalloc(&hb, sizeof(float) * (size_t)nHold * 8));
-    MCHK(hipMalloc(&hj, sizeof(float) * (size_t)nHold));
+    const int nWg = (int)std::min<long>((nHold + 31) / 32, kErrGrid);
+    float *hx = nullptr;
+    double *dPart = nullptr;
+    MCHK(hipMalloc(&hx, sizeof(float) * (size_t)nHold * 24));
+    MCHK(hipMalloc(&dPart, sizeof(double) * nWg * 24));
+    float *hy = hx + (size_t)nHold * 16;
     MCHK(hipMemcpyAsync(dIdx, hold.data(), sizeof(int) * hold.size(),
                         hipMemcpyHostToDevice, m->stream));
-    hipLaunchKernelGGL(k_gather_rows_f32, dim3((nHold + 255) / 256), dim3(256),
-                       0, m->stream, m->dataX, m->dataT, m->dataB, m->dataJ,
-                       dIdx, (int)nHold, hx, ht, hb, hj);
-    MCHK(hipStreamSynchronize(m->stream));
+    hipLaunchKernelGGL(k_gather_inputs, dim3((nHold + 15) / 16), dim3(256), 0,
+                       m->stream, m->dataX, dIdx, (int)nHold, hx);
+    MCHK(hipGetLastError());
     st = bats::mlp::forward_device(m, hx, hy, (int)nHold, m->stream);
-    std::vector<float> Y((size_t)nHold * 8), T((size_t)nHold * 8),
-        Bv((size_t)nHold * 8), Jv((size_t)nHold);
-    MCHK(hipMemcpyAsync(Y.data(), hy, sizeof(float) * Y.size(),
-                        hipMemcpyDeviceToHost, m->stream));
-    MCHK(hipMemcpyAsync(T.data(), ht, sizeof(float) * T.size(),
-                        hipMemcpyDeviceToHost, m->stream));
-    MCHK(hipMemcpyAsync(Bv.data(), hb, sizeof(float) * Bv.size(),
-                        hipMemcpyDeviceToHost, m->stream));
-    MCHK(hipMemcpyAsync(Jv.data(), hj, sizeof(float) * Jv.size(),
-                        hipMemcpyDeviceToHost, m->stream));
-    MCHK(hipStreamSynchronize(m->stream));
-    double num[9] = {0}, den[9] = {0}, denT[9] = {0};
-    for (long r = 0; r < nHold; r++)
-      for (int j = 0; j < 8; j++) {
-        // predicted flux base + w Y against the full flux base + w T,
-        // w the sample's target weight (the jump norm for harvested faces)
-        const double w = Jv[r];
-        const double d = w * ((double)Y[r * 8 + j] - (double)T[r * 8 + j]);
-        const double t = w * (double)T[r * 8 + j] + (double)Bv[r * 8 + j];
-        const double tt = w * (double)T[r * 8 + j];
-        num[j + 1] += d * d;
-        den[j + 1] += t * t;
-        denT[j + 1] += tt * tt;
-        num[0] += d * d;
-        den[0] += t * t;
-        denT[0] += tt * tt;
+    if (st == BATS_OK) {
+      hipLaunchKernelGGL(k_hold_err, dim3(nWg), dim3(256), 0, m->stream, hy,
+                         m->dataT, m->dataB, m->dataJ, dIdx, (int)nHold, dPart);
+      MCHK(hipGetLastError());
+      std::vector<double> part((size_t)nWg * 24);
+      MCHK(hipMemcpyAsync(part.data(), dPart, sizeof(double) * part.size(),
+                          hipMemcpyDeviceToHost, m->stream));
+      MCHK(hipStreamSynchronize(m->stream));
+      // sum q of output j in sum[q][j + 1], of all outputs in sum[q][0]
+      double sum[3][9] = {{0}};
+      for (int w = 0; w < nWg; w++)
+        for (int q = 0; q < 3; q++)
+          for (int j = 0; j < 8; j++)
+            sum[q][j + 1] += part[(w * 3 + q) * 8 + j];
+      for (int q = 0; q < 3; q++)
+        for (int j = 1; j < 9; j++) sum[q][0] += sum[q][j];
+      for (int j = 0; j < 9; j++) {
+        const double num = sum[0][j], den = sum[1][j], denT = sum[2][j];
+        HeldOutRelErr_V[j] = den > 0 ? sqrt(num / den) : sqrt(num);
+        HeldOutRelErr_V[9 + j] = denT > 0 ? sqrt(num / denT) : sqrt(num);
       }
-    for (int j = 0; j < 9; j++) {
-      HeldOutRelErr_V[j] = den[j] > 0 ? sqrt(num[j] / den[j]) : sqrt(num[j]);
-      HeldOutRelErr_V[9 + j] =
-          denT[j] > 0 ? sqrt(num[j] / denT[j]) : sqrt(num[j]);
     }
     (void)hipFree(hx);
-    (void)hipFree(ht);
-    (void)hipFree(hy);
-    (void)hipFree(hb);
-    (void)hipFree(hj);
+    (void)hipFree(dPart);
   }
   (void)hipFree(dIdx);
   return st;
