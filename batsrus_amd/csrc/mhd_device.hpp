@@ -373,6 +373,11 @@ template <int DIR, bool FULL, bool B0F = false, typename Real>
 __device__ __forceinline__ int hlld(const PhysT<Real> &ph, const Real *SL,
                                     const Real *SR, Real *F, Real &Cmax,
                                     Real &UnOut, const Real *B0 = nullptr) {
+  // FP32 keeps each product as the formulas have it: the surrogate's gate
+  // decides on FP32 states which flux a face takes, so that a state that
+  // differs in its last bits ends with other fluxes on some faces (two-level
+  // shear layer, Rusanov mode, 20 steps: up to 4e-3 in 100 of 300,000 cells)
+  constexpr bool FACTORS = sizeof(Real) == 8;
   constexpr int in = DIR, it1 = (DIR + 1) % 3, it2 = (DIR + 2) % 3;
   int err = 0;
   Real UnLs, FastL, UnRs, FastR;
@@ -430,12 +435,19 @@ __device__ __forceinline__ int hlld(const PhysT<Real> &ph, const Real *SL,
       Ut1L1 = Ut1L; Ut2L1 = Ut2L; B1t1L1 = B1t1L; B1t2L1 = B1t2L;
     } else {
       T = frcp(T);
-      const Real cU = Bn * (Un - UnL) * T;
-      const Real cB = (DsRhoL * DsL - Bn2) * T;
-      Ut1L1 = Ut1L - Bt1L * cU;
-      Ut2L1 = Ut2L - Bt2L * cU;
-      B1t1L1 = Bt1L * cB;
-      B1t2L1 = Bt2L * cB;
+      if constexpr (FACTORS) {
+        const Real cU = Bn * (Un - UnL) * T;
+        const Real cB = (DsRhoL * DsL - Bn2) * T;
+        Ut1L1 = Ut1L - Bt1L * cU;
+        Ut2L1 = Ut2L - Bt2L * cU;
+        B1t1L1 = Bt1L * cB;
+        B1t2L1 = Bt2L * cB;
+      } else {
+        Ut1L1 = Ut1L - Bn * Bt1L * (Un - UnL) * T;
+        Ut2L1 = Ut2L - Bn * Bt2L * (Un - UnL) * T;
+        B1t1L1 = Bt1L * (DsRhoL * DsL - Bn2) * T;
+        B1t2L1 = Bt2L * (DsRhoL * DsL - Bn2) * T;
+      }
       if (B0F) { B1t1L1 = B1t1L1 - B0t1; B1t2L1 = B1t2L1 - B0t2; }
     }
   };
@@ -445,12 +457,19 @@ __device__ __forceinline__ int hlld(const PhysT<Real> &ph, const Real *SL,
       Ut1R1 = Ut1R; Ut2R1 = Ut2R; B1t1R1 = B1t1R; B1t2R1 = B1t2R;
     } else {
       T = frcp(T);
-      const Real cU = Bn * (Un - UnR) * T;
-      const Real cB = (DsRhoR * DsR - Bn2) * T;
-      Ut1R1 = Ut1R - Bt1R * cU;
-      Ut2R1 = Ut2R - Bt2R * cU;
-      B1t1R1 = Bt1R * cB;
-      B1t2R1 = Bt2R * cB;
+      if constexpr (FACTORS) {
+        const Real cU = Bn * (Un - UnR) * T;
+        const Real cB = (DsRhoR * DsR - Bn2) * T;
+        Ut1R1 = Ut1R - Bt1R * cU;
+        Ut2R1 = Ut2R - Bt2R * cU;
+        B1t1R1 = Bt1R * cB;
+        B1t2R1 = Bt2R * cB;
+      } else {
+        Ut1R1 = Ut1R - Bn * Bt1R * (Un - UnR) * T;
+        Ut2R1 = Ut2R - Bn * Bt2R * (Un - UnR) * T;
+        B1t1R1 = Bt1R * (DsRhoR * DsR - Bn2) * T;
+        B1t2R1 = Bt2R * (DsRhoR * DsR - Bn2) * T;
+      }
       if (B0F) { B1t1R1 = B1t1R1 - B0t1; B1t2R1 = B1t2R1 - B0t2; }
     }
   };
@@ -475,12 +494,20 @@ __device__ __forceinline__ int hlld(const PhysT<Real> &ph, const Real *SL,
       const Real SqRhoR1 = fsqrt(ratio);
       outer_right();
       const Real Ti = frcp(SqRhoL1 + SqRhoR1);
-      const Real cL = SqRhoL1 * Ti, cR = SqRhoR1 * Ti, cS = SignBn * Ti;
-      const Real cLR = SqRhoL1 * SqRhoR1 * cS;
-      Ut1 = cL * Ut1L1 + cR * Ut1R1 + (B1t1R1 - B1t1L1) * cS;
-      Ut2 = cL * Ut2L1 + cR * Ut2R1 + (B1t2R1 - B1t2L1) * cS;
-      B1t1 = cL * B1t1R1 + cR * B1t1L1 + (Ut1R1 - Ut1L1) * cLR;
-      B1t2 = cL * B1t2R1 + cR * B1t2L1 + (Ut2R1 - Ut2L1) * cLR;
+      if constexpr (FACTORS) {
+        const Real cL = SqRhoL1 * Ti, cR = SqRhoR1 * Ti, cS = SignBn * Ti;
+        const Real cLR = SqRhoL1 * SqRhoR1 * cS;
+        Ut1 = cL * Ut1L1 + cR * Ut1R1 + (B1t1R1 - B1t1L1) * cS;
+        Ut2 = cL * Ut2L1 + cR * Ut2R1 + (B1t2R1 - B1t2L1) * cS;
+        B1t1 = cL * B1t1R1 + cR * B1t1L1 + (Ut1R1 - Ut1L1) * cLR;
+        B1t2 = cL * B1t2R1 + cR * B1t2L1 + (Ut2R1 - Ut2L1) * cLR;
+      } else {
+        const Real SqRhoLR1 = SqRhoL1 * SqRhoR1 * SignBn;
+        Ut1 = (SqRhoL1 * Ut1L1 + SqRhoR1 * Ut1R1 + (B1t1R1 - B1t1L1) * SignBn) * Ti;
+        Ut2 = (SqRhoL1 * Ut2L1 + SqRhoR1 * Ut2R1 + (B1t2R1 - B1t2L1) * SignBn) * Ti;
+        B1t1 = (SqRhoL1 * B1t1R1 + SqRhoR1 * B1t1L1 + (Ut1R1 - Ut1L1) * SqRhoLR1) * Ti;
+        B1t2 = (SqRhoL1 * B1t2R1 + SqRhoR1 * B1t2L1 + (Ut2R1 - Ut2L1) * SqRhoLR1) * Ti;
+      }
       uDotB1 = Un * B1n + Ut1 * B1t1 + Ut2 * B1t2;
       e = e - SqRhoL1 * (uDotB1L1 - uDotB1) * SignBn;
     }
@@ -505,12 +532,20 @@ __device__ __forceinline__ int hlld(const PhysT<Real> &ph, const Real *SL,
       const Real SqRhoL1 = fsqrt(ratio);
       outer_left();
       const Real Ti = frcp(SqRhoL1 + SqRhoR1);
-      const Real cL = SqRhoL1 * Ti, cR = SqRhoR1 * Ti, cS = SignBn * Ti;
-      const Real cLR = SqRhoL1 * SqRhoR1 * cS;
-      Ut1 = cL * Ut1L1 + cR * Ut1R1 + (B1t1R1 - B1t1L1) * cS;
-      Ut2 = cL * Ut2L1 + cR * Ut2R1 + (B1t2R1 - B1t2L1) * cS;
-      B1t1 = cL * B1t1R1 + cR * B1t1L1 + (Ut1R1 - Ut1L1) * cLR;
-      B1t2 = cL * B1t2R1 + cR * B1t2L1 + (Ut2R1 - Ut2L1) * cLR;
+      if constexpr (FACTORS) {
+        const Real cL = SqRhoL1 * Ti, cR = SqRhoR1 * Ti, cS = SignBn * Ti;
+        const Real cLR = SqRhoL1 * SqRhoR1 * cS;
+        Ut1 = cL * Ut1L1 + cR * Ut1R1 + (B1t1R1 - B1t1L1) * cS;
+        Ut2 = cL * Ut2L1 + cR * Ut2R1 + (B1t2R1 - B1t2L1) * cS;
+        B1t1 = cL * B1t1R1 + cR * B1t1L1 + (Ut1R1 - Ut1L1) * cLR;
+        B1t2 = cL * B1t2R1 + cR * B1t2L1 + (Ut2R1 - Ut2L1) * cLR;
+      } else {
+        const Real SqRhoLR1 = SqRhoL1 * SqRhoR1 * SignBn;
+        Ut1 = (SqRhoL1 * Ut1L1 + SqRhoR1 * Ut1R1 + (B1t1R1 - B1t1L1) * SignBn) * Ti;
+        Ut2 = (SqRhoL1 * Ut2L1 + SqRhoR1 * Ut2R1 + (B1t2R1 - B1t2L1) * SignBn) * Ti;
+        B1t1 = (SqRhoL1 * B1t1R1 + SqRhoR1 * B1t1L1 + (Ut1R1 - Ut1L1) * SqRhoLR1) * Ti;
+        B1t2 = (SqRhoL1 * B1t2R1 + SqRhoR1 * B1t2L1 + (Ut2R1 - Ut2L1) * SqRhoLR1) * Ti;
+      }
       uDotB1 = Un * B1n + Ut1 * B1t1 + Ut2 * B1t2;
       e = e + SqRhoR1 * (uDotB1R1 - uDotB1) * SignBn;
     }

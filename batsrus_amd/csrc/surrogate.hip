@@ -299,6 +299,16 @@ __global__ void __launch_bounds__(256) k_harvest(HarvestArgs a) {
 // ---------------------------------------------------------------------
 // surrogate stage kernels (FP32 state)
 // ---------------------------------------------------------------------
+// to_primitive with its products free to be contracted into what uses them:
+// the gate decides on these states which flux a face takes, and the products
+// rounded by themselves move a decision now and then
+__device__ __forceinline__ void face_primitive(float *q) {
+  const float RhoInv = frcp(q[RHO]);
+  q[MX] = RhoInv * q[MX];
+  q[MY] = RhoInv * q[MY];
+  q[MZ] = RhoInv * q[MZ];
+}
+
 struct SurArgs {
   const float *Uin, *Uold;
   float *Uout;
@@ -409,7 +419,7 @@ k_sur_faces(SurArgs a) {
 #pragma unroll
       for (int s = 0; s < 4; s++) load_state(a.Uin, a.vs, off[s], q[s]);
 #pragma unroll
-      for (int s = 0; s < 4; s++) to_primitive(q[s]);
+      for (int s = 0; s < 4; s++) face_primitive(q[s]);
       float L[NVAR], R[NVAR];
       face_states<LIM>(beta, beta, q[0], q[1], q[2], q[3], L, R);
       const double *cz = a.cellsize + 3 * b;
