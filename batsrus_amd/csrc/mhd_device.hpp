@@ -92,11 +92,11 @@ template <typename Real> __device__ __forceinline__ Real fdiv(Real a, Real b) {
   return a * frcp(b);
 }
 // sqrt(x), x >= 0: v_rsq_f64 + Goldschmidt refinement.  The reciprocal root
-// is taken of at least the smallest normal number, so that x = 0 gives 0
-// without a comparison and two selects.
+// is taken of x plus the smallest subnormal number, which is x itself unless
+// x is subnormal, so that x = 0 gives 0 without a comparison and two selects
+// and a negative x still gives NaN.
 __device__ __forceinline__ double fsqrt(double x) {
-  const double y =
-      __builtin_amdgcn_rsq(__builtin_fmax(x, 2.2250738585072014e-308));
+  const double y = __builtin_amdgcn_rsq(x + 4.9406564584124654e-324);
   double g = x * y, h = 0.5 * y;
   const double r = __builtin_fma(-g, h, 0.5);
   g = __builtin_fma(g, r, g);
