@@ -915,13 +915,23 @@ static int slot_threads() {
   const int n = (int)std::thread::hardware_concurrency() / 2;
   return std::min(n, kSlots);
 }
-static int ensure_slots(bats_handle *h) {
-  if (h->slotMem) return BATS_OK;
-  for (int w = 0; w < kSlots; w++)
-    if (!h->slotEv[w])
-      HIPCHK(hipEventCreateWithFlags(&h->slotEv[w], hipEventDisableTiming));
-  HIPCHK(hipHostMalloc(&h->slotMem, kSlotBytes * kSlots, 0));
-  return BATS_OK;
+// whether the handle has its slots; without pinned memory for them it never
+// asks again, and the refusal is not left behind as the thread's last error,
+// which the next launch's check would report as its own
+static bool have_slots(bats_handle *h) {
+  if (h->slotMem) return true;
+  if (h->noSlots) return false;
+  bool ok = true;
+  for (auto &ev : h->slotEv)
+    ok = ok && (ev || hipEventCreateWithFlags(&ev, hipEventDisableTiming) ==
+                          hipSuccess);
+  ok = ok && hipHostMalloc(&h->slotMem, kSlotBytes * kSlots, 0) == hipSuccess;
+  if (!ok) {
+    (void)hipGetLastError();
+    h->slotMem = nullptr;
+    h->noSlots = 1;
+  }
+  return ok;
 }
 
 // move the state through the slots: each of nThread threads takes every
@@ -1007,7 +1017,7 @@ static int copy_soa(bats_handle *h, double *host, T *state) {
   HIPCHK(hipStreamSynchronize(h->stream));
   const int nThread = slot_threads();
   if (sizeof(double) * NVAR * (size_t)h->nCell < kSlotMinBytes ||
-      nThread < 2 || ensure_slots(h) != BATS_OK)
+      nThread < 2 || !have_slots(h))
     return plain_copy<T, IN>(h, host, state);
   const int st = slot_copy<T, IN>(h, host, state, nThread);
   HIPCHK(hipStreamSynchronize(h->stream));

@@ -41,6 +41,7 @@ struct bats_handle {
   // the events of the copies through them (made on first use)
   void *slotMem;
   hipEvent_t slotEv[8];
+  int noSlots;   // no pinned memory for them: plain copies
   void *lowCrit;  // low order face weights (elemSize-byte reals,
                   // 3*NB^2*(NB+1) per block, crit_index order) or null
   int *nei;
