@@ -700,7 +700,7 @@ extern "C" int bats_init(const bats_config *cfg, bats_handle **out) {
   if (e == hipSuccess) e = hipMalloc(&h->nei, sizeof(int) * 6 * c.nBlock);
   if (e == hipSuccess) e = hipMalloc(&h->cellsize, sizeof(double) * 3 * c.nBlock);
   // the blocks' time steps and what the parts of a split block meet in:
-  // dtmaxB, dtAcc and dtCnt in one allocation, set by one copy
+  // dtmaxB, dtAcc and dtCnt in one allocation, cleared together
   const size_t nDt = c.nBlock, szDt = (2 * sizeof(double) + sizeof(unsigned)) * nDt;
   if (e == hipSuccess) e = hipMalloc(&h->dtmaxB, szDt);
   h->dtAcc = reinterpret_cast<unsigned long long *>(h->dtmaxB + nDt);
@@ -738,9 +738,7 @@ extern "C" int bats_init(const bats_config *cfg, bats_handle **out) {
                    hipMemcpyHostToDevice));
   HIPCHK(hipMemset(h->runOfBlock, 0, sizeof(int) * c.nBlock));
   HIPCHK(hipMemset(h->err, 0, sizeof(int)));
-  std::vector<double> dt0((szDt + 7) / 8, 0.0);
-  std::fill(dt0.begin() + nDt, dt0.begin() + 2 * nDt, 1.7976931348623157e308);
-  HIPCHK(hipMemcpy(h->dtmaxB, dt0.data(), szDt, hipMemcpyHostToDevice));
+  HIPCHK(hipMemset(h->dtmaxB, 0, szDt));
   h->splitShift = -1;
   // outer boundaries float until bats_set_cell_boundary
   for (int side = 0; side < 6; side++) h->bcType[side] = BATS_BC_FLOAT;

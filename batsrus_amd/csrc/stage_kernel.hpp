@@ -53,8 +53,8 @@ struct StageArgs {
   const int *runOfBlock;  // run index of each block (null: one run)
   int nRun;
   double *dtmaxB;      // per block minimum of the local time step
-  // split blocks: the minimum over the parts done so far (bit patterns,
-  // DBL_MAX between launches) and their number (0 between launches)
+  // split blocks: the minimum over the parts done so far (complement of the
+  // bit pattern) and their number, both 0 between launches
   unsigned long long *dtAcc;
   unsigned *dtCnt;
   double *dtmaxCB;     // optional per-cell local time step
@@ -1054,21 +1054,19 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
         double r = sRed[(lb * NC) / 64];
         for (int q = 1; q < WPB; q++) r = fmin2(r, sRed[(lb * NC) / 64 + q]);
         // the parts of a split block meet in an atomic minimum over the
-        // bit patterns (an order-preserving map for non-negative doubles);
-        // the last one to come takes the result and leaves the two words
-        // as it found them.  The count is raised only after the minimum
-        // has returned, so the last part sees every other one's.
+        // bit patterns (an order-preserving map for non-negative doubles),
+        // taken as the maximum of their complements so that zero is
+        // neutral; the last one to come takes the result and leaves the two
+        // words as it found them.  The count is raised only after the
+        // minimum has returned, so the last part sees every other one's.
         if (a.splitShift) {
-          const unsigned long long old =
-              atomicMin(a.dtAcc + b,
-                        (unsigned long long)__double_as_longlong(r));
+          const unsigned long long old = atomicMax(
+              a.dtAcc + b, ~(unsigned long long)__double_as_longlong(r));
           asm volatile("" ::"v"(old) : "memory");
           const unsigned last = (1u << a.splitShift) - 1;
           if (atomicInc(a.dtCnt + b, last) == last)
-            a.dtmaxB[b] = __longlong_as_double((long long)atomicExch(
-                a.dtAcc + b,
-                (unsigned long long)__double_as_longlong(
-                    1.7976931348623157e308)));
+            a.dtmaxB[b] =
+                __longlong_as_double((long long)~atomicExch(a.dtAcc + b, 0ull));
         }
         else
           a.dtmaxB[b] = r;
