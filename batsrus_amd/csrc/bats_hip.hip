@@ -1439,40 +1439,6 @@ extern "C" int bats_set_global_timestep(bats_handle *h, double TimeSimulationLim
   return BATS_OK;
 }
 
-// Parts (2^shift) into which the blocks' planes are cut when the caller sets
-// no launch shape.  A workgroup marches through its planes one behind the
-// other, about 8 us each, whatever else runs: a grid of few blocks is done
-// sooner in shorter parts, until all the places of the chip are taken (two
-// workgroups per CU in FP64, three in FP32), and a grid of a few times the
-// places ends with a nearly empty last round that shorter parts fill.  Each
-// part loads three planes more for its first face, about half a plane's
-// time.  The rule takes the least of rounds * (planes + 1/2); a last round
-// with at most one workgroup per CU takes 0.73 of a full one (FP32: 0.68,
-// with two 0.83), and beyond three rounds the workgroups no longer start
-// together, so that only the tail of the last one shows.  Measured, whole
-// blocks against the rule's parts (HLLD, per launch): FP64 8^3, 8 blocks 79
-// -> 20 us, 512 blocks 82 -> 38; 16^3, 64 blocks 143 -> 37, 105 blocks 141
-// -> 57, 256 blocks 140 -> 98, 600 blocks 336 -> 246; 512, 1000 and 4096
-// blocks stay whole (184, 381 us and 1.5 ms; in halves 186, 386 us).
-static int auto_split(int nGroup, int NB, bool f32) {
-  const int slots = f32 ? 768 : 512;
-  int best = 0;
-  double least = 0.0;
-  for (int s = 0; (NB >> s) >= 1; s++) {
-    const long items = (long)nGroup << s;
-    const long q = items / slots, rem = items % slots;
-    double rounds = (double)q;
-    if (q >= 3)
-      rounds = (double)items / slots + 0.15;
-    else if (rem > 0)
-      rounds += f32 ? (rem <= 256 ? 0.68 : rem <= 512 ? 0.83 : 1.0)
-                    : (rem <= 256 ? 0.73 : 1.0);
-    const double cost = rounds * ((NB >> s) + 0.5);
-    if (s == 0 || cost < least) { least = cost; best = s; }
-  }
-  return best;
-}
-
 // calcDt: DoCalcTimestep of the stage loop.  The local time steps are set
 // after the last stage's update (time accurate, :217-219), before the first
 // stage's update (steady state, :184-195), and always by the no-update pass.
@@ -1529,7 +1495,12 @@ static int launch_stage(bats_handle *h, int iStage, int calcDt, int noUpdate,
   // a persistent grid walks whole blocks
   const bool autoShape = h->splitShift < 0 && h->nWorkgroupMax == 0;
   const bool f32 = h->elemSize == 4;
-  a.splitShift = autoShape ? auto_split(a.nGroup, NB, f32)
+  const bool wave8 = c.UseDivbSource != 0;
+  auto parts = [&](int nGroup, bool body) {
+    return auto_split(nGroup, NB, stage_per_cu(NB, h->elemSize, wave8, body),
+                      wave8);
+  };
+  a.splitShift = autoShape ? parts(a.nGroup, false)
                            : std::max(h->splitShift, 0);
   a.dtAcc = h->dtAcc;
   a.dtCnt = h->dtCnt;
@@ -1649,9 +1620,8 @@ static int launch_stage(bats_handle *h, int iStage, int calcDt, int noUpdate,
     // workgroup per CU runs
     int bodyShift = a.splitShift;
     if (h->useBody && autoShape) {
-      bodyShift = auto_split(h->nBodyGroup, NB, f32);
-      if (h->nPlainGroup > 0)
-        a.splitShift = auto_split(h->nPlainGroup, NB, f32);
+      bodyShift = parts(h->nBodyGroup, true);
+      if (h->nPlainGroup > 0) a.splitShift = parts(h->nPlainGroup, false);
     } else if (h->useBody) {
       while ((h->nBodyGroup << bodyShift) < 256 && (NB >> (bodyShift + 1)) >= 2)
         bodyShift++;

@@ -31,6 +31,7 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include "launch_shape.hpp"
 #include "mhd_device.hpp"
 
 namespace bats {
@@ -370,10 +371,7 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
   // (three for FP32) still fit in the 160 KiB of LDS with them, and always
   // in the body variant (which changes them); otherwise the update
   // recomputes them from the plane (and the TVD faces from their records)
-  constexpr int LDS_BN = (BPW * NVAR * NR * NS + BPW * 2 * (NFS + 2) * NFX) *
-                             (int)sizeof(T) + (kThreads / 64) * 8;
-  constexpr bool BNLDS =
-      POWELL && (BODY || LDS_BN * (sizeof(T) == 4 ? 3 : 2) <= 160 * 1024);
+  constexpr bool BNLDS = stage_normal_field(NB, sizeof(T), POWELL, BODY);
   constexpr int NFL = BNLDS ? NFS + 2 : NFS;
   __shared__ T sP[BPW * NVAR * NR * NS];
   __shared__ T sF[BPW * 2 * NFL * NFX];
@@ -386,6 +384,9 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 3 : 2)
   constexpr bool AREALDS = sizeof(T) == 8 && !POWELL;
   __shared__ T sArea[AREALDS ? BPW * 2 : 1];
   __shared__ double sRed[kThreads / 64];
+  static_assert(sizeof sP + sizeof sF + sizeof sRed ==
+                    stage_lds(NB, sizeof(T), BNLDS),
+                "the launch rule counts on this LDS");
 
   // steady state: a compile-time option of the plain variants, a run-time
   // flag of the B0, body and TVD variants (which would otherwise double)
