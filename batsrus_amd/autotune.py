@@ -6,7 +6,8 @@ state, and keeps the fastest:
   * cells per thread: each thread marches NB, NB/2 or NB/4 planes of its
     column (the block's planes split over 1, 2 or 4 workgroups, which
     fills more of the chip on small grids at the price of one more z-face
-    row per part);
+    row per part), or as many as the library chooses from the number of
+    blocks (0), which is what a session that is not tuned does;
   * work order: linear, or XCD-contiguous (each of the 8 XCDs takes a
     contiguous range of the Morton-ordered work list, so neighbouring
     blocks share its L2);
@@ -81,6 +82,15 @@ def candidates(grid):
     return out
 
 
+def shapes(grid):
+    """What `tune` times: the library's own choice of the cells per thread
+    (the default of a session) in both work orders, with and without the
+    step graph, and every candidate."""
+    own = [dict(cells_per_thread=0, xcd=x, nWorkgroup=0, graph=g)
+           for x in (False, True) for g in (False, True)]
+    return own + candidates(grid)
+
+
 def apply(session, choice):
     """Set a stored choice on a session (missing keys: the defaults)."""
     session.set_persistent_grid(int(choice.get("nWorkgroup", 0)))
@@ -111,6 +121,12 @@ class Autotuner:
             json.dump(self.table, f, indent=1, sort_keys=True)
         os.replace(tmp, self.path)
 
+    def _measured(self, key):
+        """The entry of a key, unless it was measured without the library's
+        own choice among the shapes."""
+        e = self.table.get(key)
+        return e if e and e.get("own_choice_measured") else None
+
     def lookup(self, grid, scheme, nRun=1):
         return self.table.get(workload_key(grid, scheme, nRun))
 
@@ -121,13 +137,13 @@ class Autotuner:
         measured step times of every candidate."""
         nRun = 1 if runs is None else len(runs) - 1
         key = workload_key(grid, scheme, nRun)
-        if not force and key in self.table:
+        if not force and self._measured(key):
             return self.table[key]
         times = []
         with Session(grid, **scheme) as s:
             if runs is not None:
                 s.set_runs(runs)
-            for c in candidates(grid):
+            for c in shapes(grid):
                 s.upload_soa(U0)
                 s.init_timestep()
                 apply(s, c)
@@ -142,7 +158,7 @@ class Autotuner:
                     progress(times[-1])
         best = min(times, key=lambda t: t["step_us"])
         entry = dict(choice=_choice(best), step_us=best["step_us"],
-                     measured=times)
+                     own_choice_measured=True, measured=times)
         self.table[key] = entry
         self.save()
         return entry
@@ -158,16 +174,17 @@ class Autotuner:
         ncell = grids[8].nBlock * 8 ** 3
         assert grids[16].nBlock * 16 ** 3 == ncell, "not the same domain"
         key = domain_key(ncell, scheme)
-        if not force and key in self.table:
+        if not force and self._measured(key):
             return self.table[key]
-        per, shapes = {}, {}
+        per, choice = {}, {}
         for nc, g in grids.items():
             e = self.tune(g, make_state(g), scheme, nstep=nstep, warm=warm,
                           force=force, progress=progress)
             per[nc] = e["step_us"] * 1e3 / ncell
-            shapes[nc] = e["choice"]
+            choice[nc] = e["choice"]
         best = min(per, key=per.get)
-        entry = dict(choice=dict(NB=best, **shapes[best]),
+        entry = dict(choice=dict(NB=best, **choice[best]),
+                     own_choice_measured=True,
                      ns_per_cell_update={str(k): v for k, v in per.items()})
         self.table[key] = entry
         self.save()
@@ -210,8 +227,8 @@ def markdown(name, grid, scheme, entry):
     lines = ["| cells/thread | XCD order | persistent WGs | graph | step (us) |",
              "|---|---|---|---|---|"]
     for m in sorted(entry["measured"], key=lambda m: m["step_us"]):
-        lines.append("| %d | %s | %d | %s | %.1f |" % (
-            m["cells_per_thread"], "yes" if m["xcd"] else "no",
+        lines.append("| %s | %s | %d | %s | %.1f |" % (
+            m["cells_per_thread"] or "own choice", "yes" if m["xcd"] else "no",
             m["nWorkgroup"], "yes" if m["graph"] else "no", m["step_us"]))
     return "\n".join(["### %s (%s)" % (name, workload_key(grid, scheme)), "",
                       "choice: %s, %.1f us per step" % (

@@ -528,11 +528,11 @@ class Session:
                     "set_persistent_grid")
 
     def set_stage_shape(self, CellsPerThread=None, UseXcdOrder=False):
-        """Cells per thread of the stage kernel (NB, NB/2 or NB/4; None:
-        NB) and the XCD-contiguous work order (the same bits for every
-        shape).  A session without a call leaves the cells per thread to
-        the library, which chooses from the number of blocks."""
-        cpt = self.grid.nI if CellsPerThread is None else int(CellsPerThread)
+        """Cells per thread of the stage kernel (NB, NB/2 or NB/4; None or 0,
+        the default of a session: the library chooses from the number of
+        blocks) and the XCD-contiguous work order (the same bits for every
+        shape)."""
+        cpt = 0 if CellsPerThread is None else int(CellsPerThread)
         self._check(self.lib.bats_set_stage_shape(self.h, cpt,
                                                   int(bool(UseXcdOrder))),
                     "set_stage_shape")

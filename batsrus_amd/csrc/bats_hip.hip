@@ -1865,14 +1865,17 @@ extern "C" int bats_set_persistent_grid(bats_handle *h, int nWorkgroup) {
 }
 
 // cells per thread of the stage kernel (NB, NB/2 or NB/4 planes of each
-// column per work item) and the XCD-contiguous work order (the same bits)
+// column per work item, 0: by auto_split) and the XCD-contiguous work order
+// (the same bits)
 extern "C" int bats_set_stage_shape(bats_handle *h, int CellsPerThread,
                                     int UseXcdOrder) {
   if (!h) return BATS_EINVAL;
   int shift = -1;
   for (int s = 0; s <= 2; s++)
     if (CellsPerThread == (h->NB >> s)) shift = s;
-  if (shift < 0 || (UseXcdOrder != 0 && UseXcdOrder != 1)) return BATS_EINVAL;
+  if ((shift < 0 && CellsPerThread != 0) ||
+      (UseXcdOrder != 0 && UseXcdOrder != 1))
+    return BATS_EINVAL;
   drop_graphs(h);
   h->splitShift = shift;
   h->xcdOrder = UseXcdOrder;

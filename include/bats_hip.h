@@ -424,10 +424,11 @@ int bats_set_persistent_grid(bats_handle *h, int nWorkgroup);
  * (the reference fixes its loop shape at compile time: Config.pl -g and
  * the OpenACC gang/vector loops of src/ModUpdateStateFast.f90:219-311).
  * CellsPerThread = NB, NB/2 or NB/4: each block's columns are split into
- * that many planes per work item, so small grids fill more of the chip (by
- * default the library chooses from the number of blocks).  UseXcdOrder = 1 hands each of the 8 XCDs a contiguous range
- * of the work list, so neighbouring blocks share an L2.  Every shape
- * gives the same bits.  Other values return BATS_EINVAL. */
+ * that many planes per work item, so small grids fill more of the chip; 0,
+ * the default: the library chooses from the number of blocks and the kernel's
+ * variant, down to one plane.  UseXcdOrder = 1 hands each of the 8 XCDs a
+ * contiguous range of the work list, so neighbouring blocks share an L2.
+ * Every shape gives the same bits.  Other values return BATS_EINVAL. */
 int bats_set_stage_shape(bats_handle *h, int CellsPerThread, int UseXcdOrder);
 /* ------------------------------------------------------------------------
  * Learned face-flux surrogate.  No counterpart in the reference.  A small
