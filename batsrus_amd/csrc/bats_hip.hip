@@ -18,6 +18,7 @@
 #include "../../include/bats_hip.h"
 #include "stage_kernel.hpp"
 #include "handle.hpp"
+#include "transfer_way.hpp"
 
 using namespace bats;
 
@@ -900,14 +901,10 @@ static void soa_to_aos(const bats_config &c, const std::vector<int> &nei,
 // ---- host SoA (double) <-> device state buffer -----------------------
 // Large states go through pinned slots, one per host thread: a thread copies
 // (and, for an FP32 state, converts) its chunks between the caller's array
-// and its slot while the other threads' slots are on their way over PCIe.
-// One thread moves 10 to 17 GB/s of freshly allocated pageable memory, eight
-// reach 40 to 50, the link's own rate (57); a 1000-block 16^3 FP32 state
-// (262 MB on the host) takes 11 -> 6 ms up and 25 -> 7 ms down.  Below
-// kSlotMinBytes starting the threads costs more than they save.
+// and its slot while the other threads' slots are on their way over PCIe
+// (transfer_way says which).
 constexpr int kSlots = 8;
 constexpr size_t kSlotBytes = (size_t)2 << 20;
-constexpr size_t kSlotMinBytes = (size_t)8 << 20;
 
 static int slot_threads() {
   const int n = (int)std::thread::hardware_concurrency() / 2;
@@ -986,9 +983,9 @@ static int slot_copy(bats_handle *h, double *host, T *state, int nThread) {
   return status;
 }
 
-// the same without threads: one copy per variable, one synchronization
+// the same without threads, every variable in one copy
 template <typename T, bool IN>
-static int plain_copy(bats_handle *h, double *host, T *state) {
+static int one_copy(bats_handle *h, double *host, T *state) {
   const size_t n = (size_t)h->nCell;
   std::vector<T> f(sizeof(T) == 4 ? n * NVAR : 0);
   T *hp = sizeof(T) == 4 ? f.data() : reinterpret_cast<T *>(host);
@@ -1010,38 +1007,65 @@ static int plain_copy(bats_handle *h, double *host, T *state) {
   return BATS_OK;
 }
 
+// and in a blocking copy per variable
 template <typename T, bool IN>
-static int copy_soa(bats_handle *h, double *host, T *state) {
+static int each_copy(bats_handle *h, double *host, T *state) {
+  const size_t n = (size_t)h->nCell;
+  std::vector<T> f(sizeof(T) == 4 ? n : 0);
+  for (int v = 0; v < NVAR; v++) {
+    double *hv = host + v * n;
+    T *p = sizeof(T) == 4 ? f.data() : reinterpret_cast<T *>(hv);
+    if (IN) {
+      for (size_t t = 0; t < f.size(); t++) f[t] = (T)hv[t];
+      HIPCHK(hipMemcpy(state + v * h->vs, p, sizeof(T) * n,
+                       hipMemcpyHostToDevice));
+    } else {
+      HIPCHK(hipMemcpy(p, state + v * h->vs, sizeof(T) * n,
+                       hipMemcpyDeviceToHost));
+      for (size_t t = 0; t < f.size(); t++) hv[t] = (double)f[t];
+    }
+  }
+  return BATS_OK;
+}
+
+template <typename T, bool IN>
+static int copy_soa(bats_handle *h, double *host, T *state, bool written) {
   HIPCHK(hipStreamSynchronize(h->stream));
+  const TransferWay way =
+      transfer_way(NVAR * (size_t)h->nCell, sizeof(T), IN, written);
+  if (way == ONE_COPY) return one_copy<T, IN>(h, host, state);
   const int nThread = slot_threads();
-  if (sizeof(double) * NVAR * (size_t)h->nCell < kSlotMinBytes ||
-      nThread < 2 || !have_slots(h))
-    return plain_copy<T, IN>(h, host, state);
+  if (way == EACH_COPY || nThread < 2 || !have_slots(h))
+    return each_copy<T, IN>(h, host, state);
   const int st = slot_copy<T, IN>(h, host, state, nThread);
   HIPCHK(hipStreamSynchronize(h->stream));
   return st;
 }
-static int put_soa(bats_handle *h, const double *U) {
+// written: U was just written by this thread
+static int put_soa(bats_handle *h, const double *U, bool written) {
   double *host = const_cast<double *>(U);  // read only
   void *state = h->U[h->cur];
-  const int st = h->elemSize == 4
-                     ? copy_soa<float, true>(h, host, static_cast<float *>(state))
-                     : copy_soa<double, true>(h, host, static_cast<double *>(state));
+  const int st =
+      h->elemSize == 4
+          ? copy_soa<float, true>(h, host, static_cast<float *>(state), written)
+          : copy_soa<double, true>(h, host, static_cast<double *>(state),
+                                   written);
   if (st == BATS_OK) h->stateBuf = h->cur;
   return st;
 }
 static int get_soa(bats_handle *h, double *U) {
   void *state = h->U[h->stateBuf];
   return h->elemSize == 4
-             ? copy_soa<float, false>(h, U, static_cast<float *>(state))
-             : copy_soa<double, false>(h, U, static_cast<double *>(state));
+             ? copy_soa<float, false>(h, U, static_cast<float *>(state), false)
+             : copy_soa<double, false>(h, U, static_cast<double *>(state),
+                                       false);
 }
 
 extern "C" int bats_upload_state(bats_handle *h, const double *State_VGB) {
   if (!h || !State_VGB) return BATS_EINVAL;
   std::vector<double> tmp((size_t)NVAR * h->nCell);
   aos_to_soa(h->cfg, State_VGB, tmp.data());
-  return put_soa(h, tmp.data());
+  return put_soa(h, tmp.data(), true);
 }
 extern "C" int bats_download_state(bats_handle *h, double *State_VGB) {
   if (!h || !State_VGB) return BATS_EINVAL;
@@ -1053,7 +1077,7 @@ extern "C" int bats_download_state(bats_handle *h, double *State_VGB) {
 }
 extern "C" int bats_upload_state_soa(bats_handle *h, const double *U) {
   if (!h || !U) return BATS_EINVAL;
-  return put_soa(h, U);
+  return put_soa(h, U, false);
 }
 extern "C" int bats_download_state_soa(bats_handle *h, double *U) {
   if (!h || !U) return BATS_EINVAL;
