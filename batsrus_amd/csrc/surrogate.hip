@@ -384,13 +384,24 @@ k_sur_faces(SurArgs a) {
   // per wave: 64 rows of 16 inputs (BF16), then of 8 outputs (FP32)
   __shared__ __attribute__((aligned(16))) __bf16
       sRow[NET ? (kNetThreads / 64) * 64 * 16 : 8];
+  // the weights come into LDS while the first faces are evaluated
   if (NET) {
-    for (int t = threadIdx.x; t < NFRAG / 8; t += kNetThreads)
-      reinterpret_cast<bf16x8 *>(sW)[t] =
-          reinterpret_cast<const bf16x8 *>(a.frag)[t];
+    static_assert(NFRAG % 512 == 0, "whole waves of 16 bytes per lane");
+    for (int c = threadIdx.x >> 6; c < NFRAG / 512; c += blockDim.x >> 6)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void *)(
+              a.frag + c * 512 + (threadIdx.x & 63) * 8),
+          (__attribute__((address_space(3))) void *)(sW + c * 512), 16, 0, 0);
     load_biases(a.w, sBias);
-    __syncthreads();
   }
+  // every wave comes here once, with faces or without
+  bool arrived = !NET;
+  auto arrive = [&] {
+    if (arrived) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    arrived = true;
+  };
   const int lane = threadIdx.x & 63;
   __bf16 *rows = sRow + (NET ? (threadIdx.x >> 6) * 64 * 16 : 0);
   const PhysT<float> ph = phys_as<float>(a.ph);
@@ -466,6 +477,7 @@ k_sur_faces(SurArgs a) {
         F[PP] = vdt;
       }
     }
+    arrive();
     const unsigned long long mask = NET ? __ballot(net) : 0;
     if (NET && mask) {
       const int n = __popcll(mask), row = __popcll(mask & ((1ull << lane) - 1));
@@ -537,6 +549,7 @@ k_sur_faces(SurArgs a) {
 #pragma unroll
       for (int v = 0; v < NSLOT; v++) a.face[(long)v * nTot + gf] = F[v];
   }
+  arrive();
   if (NET && lane == 0 && nNet) atomicAdd(&a.counters[0], nNet);
   if (err) atomicOr(a.err, err);
 }
@@ -677,7 +690,11 @@ static void launch_harvest(int lim, int nB, hipStream_t st, const HarvestArgs &a
 
 template <int NB, bool NET>
 static void launch_sur_faces(const SurArgs &a, hipStream_t st) {
-  constexpr int threads = NET ? kNetThreads : 256;
+  // a grid that does not fill the chip's 512 places with whole workgroups
+  // takes half ones (network mode, 125 blocks of 8^3: 83 -> 79 us per step,
+  // 77 as two kernels; 343 blocks, which fill them, 119 and 135)
+  const int threads =
+      !NET ? 256 : a.nFaceTot < 512L * kNetThreads ? kNetThreads / 2 : kNetThreads;
   long nWg = (a.nFaceTot + threads - 1) / threads;
   nWg = std::min(nWg, NET ? 512L : 16384L);
   const dim3 g((unsigned)nWg), t(threads);
