@@ -231,7 +231,7 @@ k_train_rows(TrainArgs a) {
 // Weight and bias gradients of a chunk of rows (blockIdx.x): the four waves
 // share the 108 weight tiles and the 21 bias tiles (a unit row of ones times
 // dZ); every operand is 512 contiguous bytes per 16 rows, read once per wave
-// that needs it (84 KB per 32 rows and workgroup, 42 KB of it distinct).
+// that needs it (96 KB per 32 rows and workgroup, 42 KB of it distinct).
 // Bound by reading them: 26 us for 88 MB at 65,536 rows.
 __global__ void __launch_bounds__(256)
 k_train_wgrad(const bf16x4 *ops, int nPair, int perChunk, float *partial,

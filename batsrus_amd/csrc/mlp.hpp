@@ -109,10 +109,6 @@ __device__ __forceinline__ float sigmoid(float z) {
   return __builtin_amdgcn_rcpf(1.0f + __expf(-z));
 }
 __device__ __forceinline__ float silu(float z) { return z * sigmoid(z); }
-__device__ __forceinline__ float dsilu(float z) {
-  const float s = sigmoid(z);
-  return s * (1.0f + z * (1.0f - s));
-}
 
 // =====================================================================
 // batched inference: Y[rows x 8] = MLP(X[rows x 16]) with fragment-ordered

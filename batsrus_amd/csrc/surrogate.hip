@@ -323,7 +323,7 @@ struct SurArgs {
   long vs, nCellTot;
   Phys ph;
   double beta, betaMin, jumpTol, DtFactor;
-  int lim, mode, iStage, nStage, halfStep, dbTrick, doDt, roundTripOld,
+  int lim, iStage, nStage, halfStep, dbTrick, doDt, roundTripOld,
       noUpdate, advanceTime;
   float *face;     // NSLOT x nFaceTot
   long nFaceTot;   // 3 * nBlock * NF
@@ -844,7 +844,6 @@ int sur_stage(bats_handle *h, const StageArgs &sa) {
   a.jumpTol = s.jumpTol;
   a.DtFactor = sa.DtFactor;
   a.lim = sa.lim;
-  a.mode = s.mode;
   a.iStage = sa.iStage;
   a.nStage = sa.nStage;
   a.halfStep = sa.halfStep;
