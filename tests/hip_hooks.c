@@ -4,7 +4,7 @@
  *   HOOK_NO_PINNED  pinned allocations that fail as for want of memory
  *   HOOK_DEFER      copies to the device that read their source in stream
  *                   order and not before the call returns, as copies from
- *                   pinned memory do */
+ *                   pinned memory may */
 #include <dlfcn.h>
 #include <stddef.h>
 #include <stdlib.h>

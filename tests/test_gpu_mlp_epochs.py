@@ -27,4 +27,6 @@ print(hashlib.sha256(w.tobytes() + err.tobytes()).hexdigest(), loss)
 
 def test_permutations_are_copied_as_they_were():
     print("case epochs", flush=True)
-    assert hooked.run(CODE, HOOK_DEFER="1") == hooked.run(CODE)
+    want = hooked.run(CODE)
+    assert hooked.run(CODE, HOOK_DEFER="1") == want
+    assert hooked.run(CODE, HOOK_DEFER="1", HOOK_NO_PINNED="1") == want
